@@ -39,6 +39,56 @@ void hip_check(hipError_t e, const char* what)
         throw Error(AISO_ERR_HIP, std::string("HIP error in ") + what + ": " + hipGetErrorString(e));
 }
 
+// Whether a call runs on the wide kernels, by the workgroups of a launch over
+// all its shots (at most 32 are advanced together).  Time of whole calls on
+// MI355X, wide / one point per lane:
+//   free surface     0.87-0.98 from 1 shot of 200 x 400 points to 20 of 500 x 1200, every pass
+//   Born lockstep    1.01 at 80 workgroups, 0.96 at 240, 0.91-0.93 from 640 on
+//   nonlinear        1.04-1.13 to 1640 workgroups, 0.96 at 3492, 0.85-0.87 from 16000 on
+//   its adjoint      0.89-0.95 to 1968 workgroups, 1.01-1.09 from 16000 on
+//   its gradient     0.96 (8 shots of 400 x 1000)
+// The nonlinear passes of few shots are bound by each workgroup's latency,
+// which four points per lane lengthen; the adjoint's loads of v2dt2 for its
+// staged halo cost the large shapes more than the wide accesses save, and
+// the other Born passes without a free surface, whose streams of W or images
+// set their time, measured the same on either.
+static bool wide_call(const aiso_ctx* c, TileUse use, long groups)
+{
+    if (c->p.freeSurface) return true;
+    switch (use) {
+    case TileUse::Lockstep: return groups >= 160;
+    case TileUse::NlFwd: return groups >= 3000;
+    case TileUse::NlAdj: return groups < 3000;
+    case TileUse::NlGrad: return true;
+    default: return false;
+    }
+}
+
+void select_tile(aiso_ctx* c, TileUse use, int nShot)
+{
+    const bool adj = use == TileUse::Adj || use == TileUse::AdjGeneric || use == TileUse::NlAdj || use == TileUse::NlGrad;
+    const bool generic = use == TileUse::FwdGeneric || use == TileUse::AdjGeneric;
+    const FdParams& p = c->p;
+    // A caller that set a tile, a register budget or shots per workgroup
+    // chose the one-point-per-lane kernels.
+    c->wide = false;
+    if (!generic && !(adj ? c->tileAdjSet : c->tileFwdSet) && c->spb == 1 && c->occ == 6 && wide_grid_ok(p.nz, p.nx)) {
+        c->tz = kWideTZ;
+        c->tx = use == TileUse::Lockstep ? kWidePairTX : kWideTX;
+        c->wide = wide_call(c, use, (long)tiles_z(c) * tiles_x(c) * std::min(nShot, 32));
+    }
+    if (c->wide) return;
+    c->tz = adj ? c->tzAdj : c->tzFwd;
+    c->tx = adj ? c->txAdj : c->txFwd;
+    // The forward passes of the extended, tomographic and WEMVA operators
+    // run on the generic step kernel, which is faster on 32 x 32 tiles than
+    // on the specialized forward kernels' 32 x 16 (2-6 % on MI355X).
+    if (use == TileUse::FwdGeneric && !c->tileFwdSet) {
+        c->tz = 32;
+        c->tx = 32;
+    }
+}
+
 int tiles_z(const aiso_ctx* c) { return (c->p.nz - 2 * kFat + c->tz - 1) / c->tz; }
 int tiles_x(const aiso_ctx* c) { return (c->p.nx - 2 * kFat + c->tx - 1) / c->tx; }
 
@@ -257,7 +307,8 @@ void launch_timed(aiso_ctx* c, unsigned mode, int kind, const StepArgs& a, bool 
             e1 = pooled_event(c);
             c->ev.push_back({e0, e1, kind, double(c->p.interior()) * cnt});
         }
-        if (generic) HIPC(launch_step_generic(mode, c->tz, c->tx, y, lane_stream(c, l), e0, e1));
+        if (c->wide) HIPC(launch_wide(mode, c->tx, y, lane_stream(c, l), e0, e1));
+        else if (generic) HIPC(launch_step_generic(mode, c->tz, c->tx, y, lane_stream(c, l), e0, e1));
         else HIPC(launch_step(mode, c->tz, c->tx, c->spb, y, lane_stream(c, l), e0, e1, c->spb == 1 ? c->occ : 0));
     }
 }
@@ -375,8 +426,7 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
                  aiso_device* const* srcs, int nShot, aiso_device* const* recs, int nRec, int every, int mem)
 {
     const FdParams& p = c->p;
-    c->tz = c->tzAdj;
-    c->tx = c->txAdj;
+    select_tile(c, TileUse::NlGrad, nShot);
     if (!c->haveVel) throw Error(AISO_ERR_STATE, "velocity not set");
     if (nShot < 1) throw Error(AISO_ERR_PARAM, "nShot must be >= 1");
     if (nRec != 1 && nRec != nShot) throw Error(AISO_ERR_PARAM, "receiver geometry count must be 1 or nShot");
@@ -745,7 +795,7 @@ aiso_status aiso_ctx_set_tile(aiso_ctx* c, int tz, int tx)
             throw Error(AISO_ERR_PARAM, "tile must be tz in {32,64}, tx in {16,32}");
         c->tzFwd = c->tzAdj = tz;
         c->txFwd = c->txAdj = tx;
-        c->tileFwdSet = true;
+        c->tileFwdSet = c->tileAdjSet = true;
     });
 }
 
@@ -779,7 +829,7 @@ aiso_status aiso_ctx_set_option(aiso_ctx* c, const char* key, int value)
             if ((tz != 32 && tz != 64) || (tx != 16 && tx != 32))
                 throw Error(AISO_ERR_PARAM, "tile must be tz in {32,64}, tx in {16,32} (value tz*100+tx)");
             if (k == "tileFwd") { c->tzFwd = tz; c->txFwd = tx; c->tileFwdSet = true; }
-            else { c->tzAdj = tz; c->txAdj = tx; }
+            else { c->tzAdj = tz; c->txAdj = tx; c->tileAdjSet = true; }
         }
         else if (k == "batchFwd") c->batchFwd = std::max(0, value);
         else if (k == "batchAdj") c->batchAdj = std::max(0, value);

@@ -109,7 +109,8 @@ struct aiso_ctx {
     // Step-kernel tile per direction: the forward's pair kernel runs best on
     // 32 x 16 tiles, the adjoint passes on 32 x 32 (MI355X measurements).
     int tzFwd = 32, txFwd = 16, tzAdj = 32, txAdj = 32;
-    bool tileFwdSet = false;            // the caller chose the forward tile
+    bool tileFwdSet = false, tileAdjSet = false;   // the caller chose the tile
+    bool wide = false;                  // the call in progress steps on the wide kernels (wide.hip)
     int streamNT = 1;
     size_t bytesPerShot = 0;
     // work buffers
@@ -217,6 +218,12 @@ struct Request {
     int mem;
 };
 
+// What a call steps on, for its choice of tile: the kernels of the nonlinear
+// passes and their velocity gradient, the lockstep Born pass, the other Born
+// passes, or the extended and tomographic ones.
+enum class TileUse { NlFwd, NlAdj, NlGrad, Lockstep, Fwd, Adj, FwdGeneric, AdjGeneric };
+// Sets the tile of a call (c->tz, c->tx) and whether it runs on the wide kernels.
+void select_tile(aiso_ctx* c, TileUse use, int nShot);
 int tiles_z(const aiso_ctx* c);
 int tiles_x(const aiso_ctx* c);
 struct TileLists {

@@ -226,6 +226,18 @@ hipError_t launch_step(unsigned mode, int tz, int tx, int spb, const StepArgs& a
 // MODE_TOMO_*).
 hipError_t launch_step_generic(unsigned mode, int tz, int tx, const StepArgs& a, hipStream_t s,
                                hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+// The step with four z-points per lane (wide.hip), on tiles kWideTZ x tx, for
+// grids wide_grid_ok accepts.  tx == 16: MODE_NL_FWD, MODE_NL_ADJ, MODE_SRC,
+// and with a free surface MODE_SRC_WIN, MODE_BORN_SCAT, MODE_BORN_SCAT_PRE,
+// MODE_BORN_REC and MODE_REC_WIN too; tx == 32: MODE_SRC_WIN and
+// MODE_BORN_SCAT_PRE.
+constexpr int kWideTZ = 64, kWideTX = 16, kWidePairTX = 32;
+bool wide_grid_ok(int nz, int nx);
+hipError_t launch_wide(unsigned mode, int tx, const StepArgs& a, hipStream_t s, hipEvent_t e0 = nullptr,
+                       hipEvent_t e1 = nullptr);
+// The lockstep Born forward's step of both fields (launch_fwd_pair), on tiles
+// kWideTZ x kWidePairTX.
+hipError_t launch_wide_pair(const StepArgs& a, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 hipError_t launch_ring(unsigned mode, const StepArgs& a, int maxRing, hipStream_t s);
 // One fine step of every window of a launch (MODE_NL_FWD).  grid: workgroups,
 // a multiple of 8; workgroups beyond the tile count loop over further tiles

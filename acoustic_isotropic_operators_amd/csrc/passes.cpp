@@ -33,7 +33,7 @@ public:
 
 private:
     // ---- setup stages
-    void select_tile();
+    TileUse tile_use() const;
     void validate() const;
     void derive_sizes();
     void stage_operands();
@@ -115,18 +115,12 @@ private:
 
 // ------------------------------------------------------------ setup stages
 
-void Call::select_tile()
+TileUse Call::tile_use() const
 {
-    c->tz = is_adj(q.op) ? c->tzAdj : c->tzFwd;
-    c->tx = is_adj(q.op) ? c->txAdj : c->txFwd;
-    // The forward passes of the extended, tomographic and WEMVA operators
-    // run on the generic step kernel, which is faster on 32 x 32 tiles than
-    // on the specialized forward kernels' 32 x 16 (2-6 % on MI355X).
-    const bool onGeneric = is_ext(q.op) || is_tomo(q.op) || is_wemva(q.op);
-    if (!is_adj(q.op) && !c->tileFwdSet && onGeneric) {
-        c->tz = 32;
-        c->tx = 32;
-    }
+    if (is_ext(q.op) || is_tomo(q.op) || is_wemva(q.op)) return is_adj(q.op) ? TileUse::AdjGeneric : TileUse::FwdGeneric;
+    if (!is_born(q.op)) return is_adj(q.op) ? TileUse::NlAdj : TileUse::NlFwd;
+    if (q.op == Op::BornFwd && c->p.sub == 2 && c->lockstep) return TileUse::Lockstep;
+    return is_adj(q.op) ? TileUse::Adj : TileUse::Fwd;
 }
 
 void Call::validate() const
@@ -715,7 +709,7 @@ void Call::pass_lockstep()
                     pw.e0 = pooled_event(c);
                     HIPC(hipEventRecord(pw.e0, s));
                 }
-                HIPC(launch_fwd_pair(c->tz, c->tx, x, s, nullptr, nullptr));
+                HIPC(c->wide ? launch_wide_pair(x, s) : launch_fwd_pair(c->tz, c->tx, x, s));
                 ++pw.n;
             } else {
                 for (int l = 0; l < c->curLanes; ++l) {
@@ -728,8 +722,9 @@ void Call::pass_lockstep()
                         e1 = pooled_event(c);
                         c->ev.push_back({e0, e1, AISO_K_BORN_PAIR, 2.0 * double(p.interior()) * cnt});
                     }
-                    HIPC(launch_fwd_pair(c->tz, c->tx, c->curLanes > 1 ? lane_args(x, k0, cnt) : x,
-                                         lane_stream(c, l), e0, e1));
+                    const StepArgs y = c->curLanes > 1 ? lane_args(x, k0, cnt) : x;
+                    HIPC(c->wide ? launch_wide_pair(y, lane_stream(c, l), e0, e1)
+                                 : launch_fwd_pair(c->tz, c->tx, y, lane_stream(c, l), e0, e1));
                 }
             }
             bool other = ring(MODE_SRC_WIN, x);
@@ -1614,7 +1609,7 @@ void Call::outputs()
 
 void Call::run()
 {
-    select_tile();
+    select_tile(c, tile_use(), q.nShot);
     validate();
     derive_sizes();
     stage_operands();
