@@ -194,6 +194,43 @@ DevGeom* dev_geom_pair2(aiso_ctx* c, const aiso_device* d, bool region)
     return out;
 }
 
+// Sparse lists of a geometry for k_steps: with `region` every tile whose first
+// step covers a point lists it (its halo of E less one stencil), otherwise
+// only the owning tile; entries hold the LDS index of the point.
+DevGeom* dev_geom_steps(aiso_ctx* c, const aiso_device* d, int config, bool region)
+{
+    auto key = std::make_tuple(d->id, region ? -3 : -4, config);
+    auto it = c->geoms.find(key);
+    if (it != c->geoms.end()) return it->second.get();
+    auto dg = std::make_unique<DevGeom>();
+    const Geometry& g = d->g;
+    const StepsConfig& t = kStepsConfig[config];
+    const int nz = c->p.nz, nzi = nz - 2 * kFat, nxi = c->p.nx - 2 * kFat;
+    const int tZ = (nzi + t.tz - 1) / t.tz, tX = (nxi + t.tx - 1) / t.tx;
+    const int e = region ? kFat * (t.k - 1) : 0;
+    std::vector<std::vector<int2>> buckets((size_t)tZ * tX);
+    for (int r = 0; r < (int)g.regPos.size(); ++r) {
+        const int z = g.regPos[r] % nz - kFat, x = g.regPos[r] / nz - kFat;
+        if (z < 0 || z >= nzi || x < 0 || x >= nxi) continue;
+        for (int b = std::max(0, x - e) / t.tx; b <= std::min(tX - 1, (x + e) / t.tx); ++b)
+            for (int a = std::max(0, z - e) / t.tz; a <= std::min(tZ - 1, (z + e) / t.tz); ++a)
+                buckets[a + tZ * b].push_back(make_int2(steps_index(config, z - a * t.tz, x - b * t.tx), r));
+    }
+    std::vector<int> ptr(buckets.size() + 1, 0);
+    std::vector<int2> ent;
+    for (size_t i = 0; i < buckets.size(); ++i) {
+        ptr[i + 1] = ptr[i] + (int)buckets[i].size();
+        ent.insert(ent.end(), buckets[i].begin(), buckets[i].end());
+    }
+    upload(dg->tilePtr, ptr, c->stream);
+    upload(dg->ent, ent, c->stream);
+    dg->nReg = (int)g.regPos.size();
+    HIPC(hipStreamSynchronize(c->stream));
+    DevGeom* out = dg.get();
+    c->geoms.emplace(key, std::move(dg));
+    return out;
+}
+
 hipEvent_t pooled_event(aiso_ctx* c)
 {
     if (!c->evPool.empty()) {

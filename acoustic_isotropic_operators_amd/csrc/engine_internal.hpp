@@ -238,6 +238,7 @@ constexpr int kOZ2 = kPair2EZ - 2 * kFat, kOX2 = kPair2EX - 2 * kFat;
 int tiles_z2(const aiso_ctx* c);
 int tiles_x2(const aiso_ctx* c);
 DevGeom* dev_geom_pair2(aiso_ctx* c, const aiso_device* d, bool region);
+DevGeom* dev_geom_steps(aiso_ctx* c, const aiso_device* d, int config, bool region);
 
 hipEvent_t pooled_event(aiso_ctx* c);
 void wait_default_stream(aiso_ctx* c);

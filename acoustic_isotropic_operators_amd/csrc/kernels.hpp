@@ -25,6 +25,10 @@ struct ShotSlot {
     const int2* srcRing;  // (grid index, trace) for points in the FAT ring
     const int2* recRing;
     int nSrcRing, nRecRing;
+    const int* srcOwnTile;  // k_steps: the points of the tile itself, indexed like srcTile / recTile,
+    const int2* srcOwnEnt;  // which there list the points that reach its region
+    const int* recOwnTile;
+    const int2* recOwnEnt;
 };
 
 // Operating modes of the fused time-step kernel (template bits).
@@ -160,6 +164,48 @@ struct Rec2Args {
     int ntW;
 };
 
+// Up to K fine steps of a nonlinear pass per launch (k_steps): reads the
+// current and old slices p[2 pair], p[2 pair + 1] and writes the two newest
+// to p[2 (pair ^ 1)], p[2 (pair ^ 1) + 1].
+constexpr int kStepsMax = 4, kStepsPadMax = 200;    // steps per launch, sponge width
+struct StepsConfig {
+    int tz, tx, k;                  // tile and steps per launch
+};
+constexpr int kStepsConfigs = 3;
+constexpr StepsConfig kStepsConfig[kStepsConfigs] = {{32, 32, 4}, {64, 32, 3}, {64, 64, 3}};
+struct StepsArgs {
+    const ShotSlot* slots;
+    const float* v2dt2;
+    const float* cd;
+    int nz, nx, minPad, nts, ntw, nshots;
+    int tilesZ, ntiles;
+    float zc[6], xc[6];
+    int pair, n;                    // n: steps of the launch, 1 .. K
+    int its[kStepsMax];             // per step: coarse sample of the data weights wi, column of sig
+    int itw[kStepsMax];
+    float wi[kStepsMax][2];
+};
+constexpr int steps_slices(bool adj) { return adj ? 4 : 3; }   // slices in LDS
+constexpr int steps_up4(int x) { return (x + 3) / 4 * 4; }
+// The LDS copy of a TZ x TX tile and its halo of K stencils: rows -HZ .. TZ +
+// HZ - 1 and columns -E .. TX + E - 1 relative to the tile.
+template <int TZ, int TX, int K>
+struct StepsShape {
+    static constexpr int E = 5 * K, HZ = steps_up4(E), XC = TX + 2 * E;
+    static constexpr int LZ = TZ + 2 * HZ + 8 + ((TZ + 2 * HZ + 8) % 8 == 0 ? 4 : 0);
+    static constexpr int SZ = LZ * XC + 16;
+    // index of a point, from its row and column relative to the tile
+    static constexpr int index(int row, int col) { return (col + E) * LZ + HZ + 8 + row; }
+};
+// LDS index of a point of a configuration's tile, from its row and column there.
+inline int steps_index(int config, int row, int col)
+{
+    using A = StepsShape<kStepsConfig[0].tz, kStepsConfig[0].tx, kStepsConfig[0].k>;
+    using B = StepsShape<kStepsConfig[1].tz, kStepsConfig[1].tx, kStepsConfig[1].k>;
+    using C = StepsShape<kStepsConfig[2].tz, kStepsConfig[2].tx, kStepsConfig[2].k>;
+    return config == 0 ? A::index(row, col) : config == 1 ? B::index(row, col) : C::index(row, col);
+}
+
 // Shots on model windows of their own (uneven apertures): window w has its
 // own padded grid nz x nx and v^2 dtw^2; every other step parameter is
 // common.  One launch advances every tile of every window of the launch.
@@ -238,6 +284,10 @@ hipError_t launch_wide(unsigned mode, int tx, const StepArgs& a, hipStream_t s, 
 // The lockstep Born forward's step of both fields (launch_fwd_pair), on tiles
 // kWideTZ x kWidePairTX.
 hipError_t launch_wide_pair(const StepArgs& a, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+// Up to K fine steps of the nonlinear forward or adjoint (steps.hip), no
+// source or receiver in the FAT ring, no free surface.
+hipError_t launch_steps(int config, bool adj, const StepsArgs& a, hipStream_t s, hipEvent_t e0 = nullptr,
+                        hipEvent_t e1 = nullptr);
 hipError_t launch_ring(unsigned mode, const StepArgs& a, int maxRing, hipStream_t s);
 // One fine step of every window of a launch (MODE_NL_FWD).  grid: workgroups,
 // a multiple of 8; workgroups beyond the tile count loop over further tiles

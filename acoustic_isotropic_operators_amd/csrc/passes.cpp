@@ -39,6 +39,7 @@ private:
     void stage_operands();
     void build_geometry();
     void plan_batches();
+    int steps_config(int shots) const;
     void allocate();
     void prepare_model();
     void init_step_args();
@@ -48,6 +49,7 @@ private:
     void load_receiver_traces();
     void pass_pair2();
     void pass_lockstep();
+    void pass_steps();
     void pass_adjoint2();
     void pass_source();
     void passes_tomo();
@@ -79,6 +81,7 @@ private:
     int nExt = 1, nImg = 1, nRecDev = 0, nSrcDev = 0, h = 0;
     const float* f = nullptr;
     bool wemva = false, tomo = false, perShotImg = false, dataInput = false, fsurf = false, tlag = false;
+    int steps = -1;                     // k_steps configuration of the call, or -1
     bool lockstep = false, pair2 = false, adj2 = false, win = false, generic = false;
     bool needW = false, needSS = false, needImg = false;
     int pairSlices = 2, ssSlices = 2, capSlices = 2, extK = 1, B = 1;
@@ -266,7 +269,12 @@ void Call::plan_batches()
     for (int i = 0; noRing && i < q.nRec; ++i) noRing = recG[i]->nRing == 0;
     pair2 = lockstep && c->pair2 && noRing && !fsurf;
     adj2 = q.op == Op::BornAdj && p.sub == 2 && c->pair2 && noRing && !fsurf;
-    pairSlices = pair2 || adj2 ? 4 : 2;
+    // Several steps per launch (k_steps) where few workgroups carry the call.
+    const bool tileSet = is_adj(q.op) ? c->tileAdjSet : c->tileFwdSet;
+    bool multi = !is_born(q.op) && noRing && !fsurf && !tileSet && c->spb == 1 && c->occ == 6 &&
+                 p.minPad <= kStepsPadMax && wide_grid_ok(p.nz, p.nx);
+    multi = multi && steps_config(1) >= 0;
+    pairSlices = pair2 || adj2 || multi ? 4 : 2;
     wSlices = lockstep ? 3 : p.nts;
     needW = is_born(q.op);
     needSS = is_ext(q.op) || tomo || q.op == Op::BornAdj;
@@ -323,6 +331,28 @@ void Call::plan_batches()
     B = std::min(B, q.nShot);
     B = (q.nShot + (q.nShot + B - 1) / B - 1) / ((q.nShot + B - 1) / B);   // same batch count, balanced sizes
     c->batchUsed = B;
+    steps = multi ? steps_config(B) : -1;
+    if (multi && steps < 0) {
+        pairSlices = 2;
+        c->bytesPerShot -= 2 * nzx * 4;
+    }
+}
+
+// The tiles and steps per launch with which `shots` shots run on k_steps: the
+// smallest tile whose workgroups all run at once, one per CU, or for the
+// forward two rounds of the largest; -1: none, and the one-step kernels are
+// faster.  Microseconds per step with the largest tile and in one-step
+// launches: 304 x 512 points, 8 shots, 320 workgroups: forward 6.3 against
+// 7.8; 608 x 1312, 2 shots, 400 workgroups: forward 7.3 against 7.8; 400 x
+// 768, 6 shots, 504 workgroups: adjoint 8.4 against 7.4.
+int Call::steps_config(int shots) const
+{
+    for (int i = 0; i < kStepsConfigs; ++i) {
+        const StepsConfig& t = kStepsConfig[i];
+        const long n = (long)((p.nz - 2 * kFat + t.tz - 1) / t.tz) * ((p.nx - 2 * kFat + t.tx - 1) / t.tx) * shots;
+        if (n <= (i + 1 < kStepsConfigs || is_adj(q.op) ? 256 : 512)) return i;
+    }
+    return -1;
 }
 
 void Call::allocate()
@@ -504,7 +534,7 @@ void Call::begin_batch(int first, int count)
     a = base;
     a.nshots = nb;
     a.gridLogical = a.ntiles * nb;
-    c->curLanes = pair2 || adj2 ? 1 : std::max(1, std::min(c->lanes, nb));
+    c->curLanes = pair2 || adj2 || steps >= 0 ? 1 : std::max(1, std::min(c->lanes, nb));
     if (c->curLanes > 1) ensure_lanes(c);
 }
 
@@ -556,6 +586,23 @@ void Call::upload_tables()
     if (tomo) bytes += 2 * stage_size(tb);
     if (q.op == Op::WemvaFwd) bytes += 2 * stage_size(tb);
     if (sigUp) bytes += stage_size(sigHost.size() * 4);
+    if (steps >= 0) {
+        for (int k = 0; k < nb; ++k) {
+            const aiso_device *src = q.src[b0 + k], *rec = rec_dev(b0 + k);
+            auto set = [&](const aiso_device* d, bool region, const int*& ptr, const int2*& ent) {
+                DevGeom* g = dev_geom_steps(c, d, steps, region);
+                ptr = g->tilePtr.as<int>();
+                ent = g->ent.as<int2>();
+            };
+            if (is_adj(q.op)) {
+                set(rec, true, slots[k].recTile, slots[k].recEnt);
+                set(src, false, slots[k].srcOwnTile, slots[k].srcOwnEnt);
+            } else {
+                set(src, true, slots[k].srcTile, slots[k].srcEnt);
+                set(rec, false, slots[k].recOwnTile, slots[k].recOwnEnt);
+            }
+        }
+    }
     stage_begin(c, bytes);
     stage_copy(c, dSlots, slots.data(), tb);
     if (!slotsQ.empty()) stage_copy(c, dSlotsQ, slotsQ.data(), tb);
@@ -1201,6 +1248,43 @@ void Call::passes_tomo()
     }
 }
 
+// The nonlinear propagation, forward or adjoint, several fine steps per launch.
+void Call::pass_steps()
+{
+    HIPC(launch_fill(pairs, (long)nb * 4 * nzx, s));
+    const bool adj = is_adj(q.op);
+    const int kind = adj ? AISO_K_NL_ADJ : AISO_K_NL_FWD, T = p.ntw - 1;
+    const StepsConfig& t = kStepsConfig[steps];
+    StepsArgs x{};
+    x.slots = dSlots;
+    x.v2dt2 = base.v2dt2;
+    x.cd = base.cd;
+    x.nz = p.nz; x.nx = p.nx; x.minPad = p.minPad; x.nts = p.nts; x.ntw = p.ntw;
+    x.nshots = nb;
+    x.tilesZ = (p.nz - 2 * kFat + t.tz - 1) / t.tz;
+    x.ntiles = x.tilesZ * ((p.nx - 2 * kFat + t.tx - 1) / t.tx);
+    for (int k = 0; k < 6; ++k) { x.zc[k] = p.zc[k]; x.xc[k] = p.xc[k]; }
+    for (int done = 0; done < T; done += x.n) {
+        x.n = std::min(t.k, T - done);
+        for (int i = 0; i < x.n; ++i) {
+            const int itw = adj ? T - 1 - done - i : done + i, it2 = itw % p.sub;
+            x.itw[i] = itw;
+            x.its[i] = itw / p.sub;
+            x.wi[i][0] = f[it2 + 1];
+            x.wi[i][1] = f[h + it2 + 1];
+        }
+        hipEvent_t e0 = nullptr, e1 = nullptr;
+        if (sample_event(c, kind)) {
+            e0 = pooled_event(c);
+            e1 = pooled_event(c);
+            c->ev.push_back({e0, e1, kind, double(p.interior()) * nb * x.n});
+        }
+        HIPC(launch_steps(steps, adj, x, s, e0, e1));
+        x.pair ^= 1;
+    }
+    if (!adj) record_data();
+}
+
 // Second pass of the forward operators: the nonlinear propagation, or the
 // Born / extended-Born scattered field, with the data recorded.
 void Call::pass_forward()
@@ -1628,7 +1712,8 @@ void Call::run()
         if (is_born(q.op) && !lockstep && !adj2) pass_source();
         if (tomo) passes_tomo();
         if (!lockstep && !adj2 && !tomo) {
-            if (q.op == Op::NlFwd || q.op == Op::BornFwd || q.op == Op::ExtFwd) pass_forward();
+            if (steps >= 0) pass_steps();
+            else if (q.op == Op::NlFwd || q.op == Op::BornFwd || q.op == Op::ExtFwd) pass_forward();
             else pass_adjoint();
         }
         reduce_images();

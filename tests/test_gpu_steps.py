@@ -1,0 +1,67 @@
+"""The kernels that take several fine steps of a nonlinear pass per launch give
+the float oracle's results bit for bit: interior sizes that leave remainders
+of their 32 x 32, 64 x 32 and 64 x 64 tiles, step counts that are no multiple
+of the steps per launch, sources and receivers on both sides of tile edges
+and inside a neighbour's halo, sponges narrower and wider than a tile, more
+receivers on a tile than it has threads, and shot counts on both sides of
+the ones at which the tile changes."""
+import numpy as np
+import pytest
+
+from cases import make_case
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+FAT = 5
+
+
+def _check(nzi, nxi, shots, sub, nts, pad, points):
+    from acoustic_isotropic_operators_amd import _capi as A
+    c = make_case(seed=nzi * 7 + nxi, nz=nzi + 2 * FAT, nx=nxi + 2 * FAT, nShot=shots, nts=nts, sub=sub, pad=pad,
+                  dts=0.001 * sub)
+    ctx = A.Context(dict(nz=c.nz, nx=c.nx, dz=c.dz, dx=c.dx, nts=c.nts, dts=c.dts, sub=c.sub, alphaCos=c.alpha,
+                         fMax=20.0, zPadMinus=pad, zPadPlus=pad, xPadMinus=pad, xPadPlus=pad))
+    ctx.set_velocity(c.vel)
+    g = c.grid
+    rng = np.random.default_rng(9)
+    # sources next to tile edges, receivers as asked for
+    at = [(FAT + min(nzi - 1, 31 + s % 3), FAT + (s * 31 + 30) % nxi) for s in range(shots)]
+    if points == "all":
+        iz, ix = (v.ravel().tolist() for v in np.mgrid[FAT:FAT + nzi, FAT:FAT + nxi])
+    else:
+        iz = [FAT, FAT + nzi - 1] + [FAT + (17 * k) % nzi for k in range(points)]
+        ix = [FAT, FAT + nxi - 1] + [FAT + (5 * k) % nxi for k in range(points)]
+        iz, ix = (list(v) for v in zip(*sorted(set(zip(iz, ix)))))
+    dims = (c.nz, c.nx, c.nts)
+    srcs = [A.Device.ints([z], [x], *dims) for z, x in at]
+    osrc = [O.Device.ints([z], [x], *dims) for z, x in at]
+    recs, orec = [A.Device.ints(iz, ix, *dims)], [O.Device.ints(iz, ix, *dims)]
+    w = rng.standard_normal((shots, 1, nts)).astype(np.float32)
+    d = np.zeros((shots, len(iz), nts), np.float32)
+    ctx.nl_forward(w, d, srcs, recs)
+    ref = O.nl_forward(g, c.vel, osrc, orec, w, "f")
+    assert np.abs(ref).max() > 0
+    np.testing.assert_array_equal(d, ref)
+    dr = rng.standard_normal(d.shape).astype(np.float32)
+    m = np.zeros((shots, 1, nts), np.float32)
+    ctx.nl_adjoint(m, dr, srcs, recs)
+    np.testing.assert_array_equal(m, O.nl_adjoint(g, c.vel, osrc, orec, dr, shots, "f"))
+
+
+@pytest.mark.parametrize("nzi,nxi,shots,sub,nts,pad", [
+    (32, 32, 1, 2, 2, 10),         # one tile, two steps
+    (48, 80, 1, 4, 12, 10),        # remainders of 16
+    (64, 96, 2, 3, 18, 4),         # 51 steps: a last launch of 3
+    (112, 80, 1, 1, 40, 40),       # sponge wider than a tile, 39 steps
+    (208, 240, 6, 2, 20, 10),      # 64 x 32 tiles, 38 steps: a last launch of 2
+    (208, 240, 14, 2, 21, 10),     # 64 x 64 tiles, 40 steps: a last launch of 1
+    (208, 256, 26, 4, 8, 50),      # 416 workgroups, two rounds
+    (272, 304, 24, 2, 12, 10),     # one step per launch again
+])
+def test_nonlinear_passes(nzi, nxi, shots, sub, nts, pad):
+    _check(nzi, nxi, shots, sub, nts, pad, 37)
+
+
+def test_more_receivers_than_threads():
+    _check(64, 64, 1, 2, 9, 10, "all")
+    _check(64, 64, 60, 2, 5, 10, "all")
