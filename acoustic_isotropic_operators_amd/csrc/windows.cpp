@@ -69,6 +69,8 @@ struct aiso_batch {
     int nSrcDev = 0;
     // the configuration the device tables hold, and the graphs captured with it
     aiso::BatchConfig cfg, prepared;
+    bool cfgSet = false;              // cfg was set or tuned; else the tile width of the tables is chosen here
+    int tx = 0;                       // tile width of the device tables
     bool isPrepared = false;
     std::vector<int> groupTiles;      // tiles of each launch group
     std::vector<long> groupPts;       // interior points of each launch group
@@ -125,10 +127,24 @@ int n_groups(const aiso_batch* b, const BatchConfig& c)
     return (n + spl - 1) / spl;
 }
 
-// Device tables of configuration c: slots, window descriptors, tile map.
-void prepare(aiso_batch* b, const BatchConfig& c)
+// Tile width of a batch whose configuration the caller left open.  A 32 x 32
+// tile reads 1.6 times its points to stage the halo, a 32 x 16 tile 2.1 times,
+// but makes twice the workgroups, which few points need.  Time of 300 samples
+// on 32 x 32 / 32 x 16 tiles (MI355X): 24 windows of 400 x 300-1500 points 19.7 /
+// 22.6 ms, 40 of 287 x 900 17.4 / 20.3 ms; 3 of 400 x 1500 (1600 tiles of 32 x 32)
+// 4.61 / 4.54 ms, 6 of 150 x 700 (830) 3.61 / 3.42 ms.
+int open_tile_width(const aiso_batch* b)
 {
-    if (b->isPrepared && b->prepared == c) return;
+    long tiles = 0;
+    for (auto& W : b->win) tiles += window_tiles(W->p, 32, 32);
+    return tiles >= 4096 ? 32 : 16;
+}
+
+// Device tables of configuration c: slots, window descriptors, tile map.
+void prepare(aiso_batch* b, const BatchConfig& c, bool set)
+{
+    const int tx = set ? c.tx : open_tile_width(b);
+    if (b->isPrepared && b->prepared == c && b->tx == tx) return;
     if (c.tz != 32 && c.tz != 64) throw Error(AISO_ERR_PARAM, "tile tz must be 32 or 64");
     if (c.tx != 16 && c.tx != 32) throw Error(AISO_ERR_PARAM, "tile tx must be 16 or 32");
     if (c.spl < 0 || c.persist < 0) throw Error(AISO_ERR_PARAM, "windows per launch and workgroups per CU are >= 0");
@@ -145,8 +161,8 @@ void prepare(aiso_batch* b, const BatchConfig& c)
         long pts = 0;
         for (int w = g0; w < std::min(n, g0 + spl); ++w) {
             aiso_batch::Win& W = *b->win[w];
-            WinGeom* sg = win_geom(b, W, W.src, true, c.tz, c.tx);
-            WinGeom* rg = win_geom(b, W, W.rec, false, c.tz, c.tx);
+            WinGeom* sg = win_geom(b, W, W.src, true, c.tz, tx);
+            WinGeom* rg = win_geom(b, W, W.rec, false, c.tz, tx);
             ShotSlot& S = slots[w];
             std::memset(&S, 0, sizeof(S));
             S.p[0] = b->pairs.as<float>() + b->pairOff[w];
@@ -162,7 +178,7 @@ void prepare(aiso_batch* b, const BatchConfig& c)
             D.nz = W.p.nz;
             D.nx = W.p.nx;
             D.tilesZ = (W.p.nz - 2 * kFat + c.tz - 1) / c.tz;
-            D.ntiles = (int)window_tiles(W.p, c.tz, c.tx);
+            D.ntiles = (int)window_tiles(W.p, c.tz, tx);
             for (int t = 0; t < D.ntiles; ++t) map.push_back(make_int2(w - g0, t));
             tiles += D.ntiles;
             pts += W.interior();
@@ -175,6 +191,7 @@ void prepare(aiso_batch* b, const BatchConfig& c)
     upload(b->tileMap, map, b->stream);
     HIPC(hipStreamSynchronize(b->stream));   // the host vectors go out of scope
     b->prepared = c;
+    b->tx = tx;
     b->isPrepared = true;
     b->graphs.assign(b->groupTiles.size(), nullptr);
 }
@@ -269,7 +286,7 @@ void launch_steps(aiso_batch* b, int g, int t0, int t1, hipStream_t st, hipEvent
         w.a.ff = f[h + it2];
         hipEvent_t a0 = t == t0 ? e0 : nullptr, a1 = t == t1 - 1 ? e1 : nullptr;
         if (a0 && !a1) HIPC(hipEventRecord(a0, st));
-        HIPC(launch_step_windows(MODE_NL_FWD, b->prepared.tz, b->prepared.tx, grid, w, st,
+        HIPC(launch_step_windows(MODE_NL_FWD, b->prepared.tz, b->tx, grid, w, st,
                                  a0 && a1 ? a0 : nullptr, a0 && a1 ? a1 : nullptr));
         if (a1 && !a0) HIPC(hipEventRecord(a1, st));
     }
@@ -350,7 +367,7 @@ void batch_nl_forward(aiso_batch* b, int add, const float* const* model, int nMo
         HIPC(hipEventRecord(b->evIn, nullptr));
         HIPC(hipStreamWaitEvent(s, b->evIn, 0));
     }
-    prepare(b, b->cfg);
+    prepare(b, b->cfg, b->cfgSet);
     const FdParams& p0 = b->win[0]->p;
     const size_t modelN = (size_t)b->nSrcDev * p0.nts;
     // source traces of every window, staged through pinned memory
@@ -411,7 +428,7 @@ void batch_nl_forward(aiso_batch* b, int add, const float* const* model, int nMo
 // point-update.
 double time_config(aiso_batch* b, const BatchConfig& c, int steps)
 {
-    prepare(b, c);
+    prepare(b, c, true);
     const int G = (int)b->groupTiles.size();
     const int L = lanes_for(b, c, G);
     hipStream_t s = b->stream;
@@ -557,6 +574,7 @@ aiso_status aiso_batch_set_config(aiso_batch* b, int tz, int tx, int windowsPerL
         if (windowsPerLaunch < 0 || blocksPerCU < 0) throw Error(AISO_ERR_PARAM, "negative configuration value");
         if (lanes < 1 || lanes > 4) throw Error(AISO_ERR_PARAM, "lanes must be 1..4");
         b->cfg = BatchConfig{tz, tx, windowsPerLaunch, blocksPerCU, lanes};
+        b->cfgSet = true;
         if (graph != b->useGraph) {
             HIPC(hipSetDevice(b->device));
             HIPC(hipStreamSynchronize(b->stream));
@@ -620,6 +638,7 @@ aiso_status aiso_batch_tune(aiso_batch* b, int steps, double* msPerPointUpdate)
         const auto best = *std::min_element(cand.begin(), cand.end(),
                                             [](const auto& x, const auto& y) { return x.first < y.first; });
         b->cfg = best.second;
+        b->cfgSet = true;
         if (msPerPointUpdate) *msPerPointUpdate = best.first;
     });
 }
