@@ -454,11 +454,15 @@ aiso_status guard(F&& f)
 // has as transpose the nonlinear adjoint propagation; driven by dJ/dd its
 // damped slices nu_t give dJ/dv2dt2 = sum_t (L p_{t-1}) * nu_t, plus at the
 // source points sum_t nu_t * u_t for the v2dt2 factor of the injected source
-// s = v2dt2 * u.  The forward slices are recomputed backward in segments of
-// K steps from checkpoints (the pair of slices every K steps).  Per batch of
-// shots: one forward pass writing checkpoints, then per segment, last first,
-// a forward recompute into W (K slices) and the K adjoint steps, each
-// followed by the imaging kernel.
+// s = v2dt2 * u.  Time is cut into segments of K steps.  Per batch of shots:
+// one forward pass that writes a checkpoint (the pair of slices) at the start
+// of each segment but the last, whose L p_{t-1} it keeps in W (K slices);
+// then per segment, last first, the recompute of its forward steps into W
+// (but for the last) and its K adjoint steps, which image against W.  The
+// one-point-per-lane kernels keep p_{t-1} itself and image in a kernel of its
+// own, which makes the Laplacian again; with them every segment is
+// recomputed.  Misfit and gradient of 8 shots of 400 x 1000 points, 800 samples
+// (MI355X): 132 ms with those and K = 40, 95 ms with one segment.
 void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dataGrad, float* velGrad,
                  aiso_device* const* srcs, int nShot, aiso_device* const* recs, int nRec, int every, int mem)
 {
@@ -482,9 +486,6 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
     const long nzx = p.nzx();
     const int h = p.h(), T = p.ntw - 1;
     const float* f = p.filt.data();
-    const int K = every > 0 ? std::min(every, T) : std::max(1, (int)std::ceil(std::sqrt((double)T)));
-    const int nCk = (T - 1) / K + 1;                   // checkpoints at t = 0, K, 2K, ... < T
-
     std::vector<float> hModel((size_t)nShotSig * nSrcDev * p.nts);
     if (mem == AISO_MEM_DEVICE) HIPC(hipMemcpy(hModel.data(), model, hModel.size() * 4, hipMemcpyDeviceToHost));
     else std::memcpy(hModel.data(), model, hModel.size() * 4);
@@ -509,26 +510,41 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
     for (auto* g : srcG) maxSrcRing = std::max(maxSrcRing, g->nRing);
     for (auto* g : recG) maxRecRing = std::max(maxRecRing, g->nRing);
 
-    // per shot: forward pair, adjoint pair, K segment slices, gradient, checkpoints
-    const size_t perShot = (size_t)(2 + 2 + K + 1 + 2 * nCk) * nzx * 4 + (size_t)nRecRegMax * p.nts * 4 +
-                           2 * (size_t)nSrcRegMax * p.ntw * 4;
+    // The wide kernels keep the Laplacian of each forward slice while they step
+    // it, and image the adjoint slices as they make them; the imaging kernel
+    // (k_grad), which makes the Laplacian again, takes it from slices without
+    // the sources of the FAT ring.
+    const bool fused = c->wide && maxSrcRing == 0;
     // 16 shots per batch by default, 8 per lane: at 400 x 1000 with 8 per
     // batch a lane's launch covers the GPU about once (MI355X: 230 against
     // 254 Gpts/s for 16; 12 and 32 gave 249 and 251).
     int B = c->batchAdj > 0 ? c->batchAdj : (c->batchReq > 0 ? c->batchReq : 16);
-    {
-        size_t freeB = 0, totalB = 0;
-        HIPC(hipMemGetInfo(&freeB, &totalB));
-        size_t have = c->pairs.n + c->pairsQ.n + c->W.n + c->img.n + c->dreg.n + c->sig.n + c->ss.n + c->ck.n;
-        B = std::min(B, (int)std::max<size_t>(1, (size_t)((freeB + have) * 0.85) / perShot));
+    size_t freeB = 0, totalB = 0;
+    HIPC(hipMemGetInfo(&freeB, &totalB));
+    freeB += c->pairs.n + c->pairsQ.n + c->W.n + c->img.n + c->dreg.n + c->sig.n + c->ss.n + c->ck.n;
+    // Steps per segment.  Every segment but the last is propagated twice, so
+    // the fused kernels take as few as a quarter of the free memory, at most
+    // 64 GB, holds slices for (one where it holds every step's).
+    int K = every > 0 ? std::min(every, T) : std::max(1, (int)std::ceil(std::sqrt((double)T)));
+    if (every == 0 && fused) {
+        const size_t cap = std::min<size_t>(freeB / 4, (size_t)64 << 30);
+        const long fit = (long)(cap / ((size_t)std::min(B, nShot) * nzx * 4));
+        const int Kmax = (int)std::min<long>(T, std::max<long>(K, fit)), segments = (T + Kmax - 1) / Kmax;
+        K = (T + segments - 1) / segments;
     }
+    const int nSeg = (T - 1) / K + 1;                  // segments start at t = 0, K, 2K, ... < T
+    const int nCk = fused ? nSeg - 1 : nSeg;           // of which these are started from checkpoints
+    // per shot: forward pair, adjoint pair, K segment slices, gradient, checkpoints
+    const size_t perShot = (size_t)(2 + 2 + K + 1 + 2 * nCk) * nzx * 4 + (size_t)nRecRegMax * p.nts * 4 +
+                           2 * (size_t)nSrcRegMax * p.ntw * 4;
+    B = std::min(B, (int)std::max<size_t>(1, (size_t)(freeB * 0.85) / perShot));
     B = std::min(B, nShot);
     c->batchUsed = B;
     float* pairs = (float*)c->pairs.need((size_t)B * 2 * nzx * 4);
     float* pairsA = (float*)c->pairsQ.need((size_t)B * 2 * nzx * 4);
     float* W = (float*)c->W.need((size_t)B * K * nzx * 4);
     float* img = (float*)c->img.need((size_t)B * nzx * 4);
-    float* ck = (float*)c->ck.need((size_t)B * 2 * nCk * nzx * 4);
+    float* ck = nCk > 0 ? (float*)c->ck.need((size_t)B * 2 * nCk * nzx * 4) : nullptr;
     float* dreg = (float*)c->dreg.need((size_t)B * nRecRegMax * p.nts * 4);
     float* sig = (float*)c->sig.need((size_t)B * nSrcRegMax * p.ntw * 4);
     float* sigA = (float*)c->ss.need((size_t)B * nSrcRegMax * p.ntw * 4);
@@ -606,7 +622,7 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
         HIPC(launch_fill(pairsA, (long)nb * 2 * nzx, s));
         // The recompute writes interior points only; the imaging kernel's
         // Laplacian reads the FAT ring of these slices, which must hold 0.
-        HIPC(launch_fill(W, (long)nb * K * nzx, s));
+        if (!fused) HIPC(launch_fill(W, (long)nb * K * nzx, s));
 
         StepArgs a = base;
         a.nshots = nb;
@@ -638,7 +654,7 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
             }
         };
         // forward: one fine step = MODE_SRC without capture (step, injection, sponge)
-        auto fwd_step = [&](int t, int cur, long capture) {
+        auto fwd_step = [&](int t, int cur, long capture, unsigned mode = MODE_SRC) {
             StepArgs x = a;
             x.slots = dF;
             x.cur = cur;
@@ -650,36 +666,46 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
             x.wA = capture >= 0 ? capture : 0;
             x.assignB = 0;
             x.skipB = 1;
-            launch_timed(c, MODE_SRC, AISO_K_SRC, x);
+            launch_timed(c, mode, AISO_K_SRC, x);
             if (maxSrcRing > 0) ring_lanes(M_INJ_SIG, x, maxSrcRing);
         };
         c->curLanes = std::max(1, std::min(c->lanes, nb));
         if (c->curLanes > 1) ensure_lanes(c);
         fork_lanes(c);
         int cur = 1;
-        save(0, cur);
-        for (int t = 1; t < T; ++t) {
+        const int tLast = (nSeg - 1) * K;              // the fused pass goes on into the last segment
+        if (nCk > 0) save(0, cur);
+        for (int t = 1; t < (fused ? tLast + 1 : T); ++t) {
             fwd_step(t, cur, -1);
             cur ^= 1;
-            if (t % K == 0) save(t / K, cur);
+            if (t % K == 0 && t / K < nCk) save(t / K, cur);
         }
         // backward, segment by segment
         StepArgs r = a;
         r.slots = dA;
         r.cur = 1;
         ga.slots = dA;
-        for (int j = nCk - 1; j >= 0; --j) {
+        for (int j = nSeg - 1; j >= 0; --j) {
             const int t0 = j * K, t1 = std::min(t0 + K, T);
-            for (int k = 0; k < nb; ++k) {
-                hipStream_t ls = lane_of(k);
-                HIPC(hipMemcpyAsync(fs[k].p[1], ckSlice(k, j, 0), nzx * 4, hipMemcpyDeviceToDevice, ls));
-                HIPC(hipMemcpyAsync(fs[k].p[0], ckSlice(k, j, 1), nzx * 4, hipMemcpyDeviceToDevice, ls));
-                HIPC(hipMemcpyAsync(fs[k].W, ckSlice(k, j, 0), nzx * 4, hipMemcpyDeviceToDevice, ls));
+            if (j < nCk) {
+                for (int k = 0; k < nb; ++k) {
+                    hipStream_t ls = lane_of(k);
+                    HIPC(hipMemcpyAsync(fs[k].p[1], ckSlice(k, j, 0), nzx * 4, hipMemcpyDeviceToDevice, ls));
+                    HIPC(hipMemcpyAsync(fs[k].p[0], ckSlice(k, j, 1), nzx * 4, hipMemcpyDeviceToDevice, ls));
+                    if (!fused) HIPC(hipMemcpyAsync(fs[k].W, ckSlice(k, j, 0), nzx * 4, hipMemcpyDeviceToDevice, ls));
+                }
+                cur = 1;
             }
-            int fc = 1;
-            for (int t = t0 + 1; t < t1; ++t) {          // W[t - t0] = p_t
-                fwd_step(t, fc, (long)(t - t0) * nzx);
-                fc ^= 1;
+            if (fused) {
+                for (int t = t0 + 1; t <= t1; ++t) {     // W[t - 1 - t0] = L(p_{t-1}), p_t
+                    fwd_step(t, cur, (long)(t - 1 - t0) * nzx, MODE_SRC_LAP);
+                    cur ^= 1;
+                }
+            } else {
+                for (int t = t0 + 1; t < t1; ++t) {      // W[t - t0] = p_t
+                    fwd_step(t, cur, (long)(t - t0) * nzx);
+                    cur ^= 1;
+                }
             }
             for (int t = t1; t > t0; --t) {              // nu_t, then img += L(p_{t-1}) nu_t
                 const int itw = t - 1, its = itw / p.sub, it2 = itw % p.sub;
@@ -687,10 +713,12 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
                 r.itwRec = itw;
                 r.fc = f[it2 + 1];
                 r.fd = f[h + it2 + 1];
-                launch_timed(c, MODE_NL_ADJ, AISO_K_NL_ADJ, r);
+                r.wImg = (long)(t - 1 - t0) * nzx;
+                launch_timed(c, fused ? MODE_ADJ_GRAD : MODE_NL_ADJ, AISO_K_NL_ADJ, r);
                 if (maxSrcRing > 0 || maxRecRing > 0)
                     ring_lanes(M_INJ_DATA | M_REC_SIG, r, std::max(maxSrcRing, maxRecRing));
                 r.cur ^= 1;
+                if (fused) continue;
                 ga.wF = (long)(t - 1 - t0) * nzx;
                 ga.nu = r.cur;
                 for (int l = 0; l < c->curLanes; ++l) {

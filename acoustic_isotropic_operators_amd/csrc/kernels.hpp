@@ -46,6 +46,8 @@ enum : unsigned {
     M_SS_PRE = 1u << 10,    // + SS[a]*fa + SS[b]*fb, SS = m~*W stored in the W array
     M_CAP_W = 1u << 11,     // adjoint stepper: capture into W[wA], W[wB] instead of ss
     M_CAP_ALT = 1u << 12,   // forward stepper: capture into img[wA], img[wB] instead of W
+    M_LAP = 1u << 13,       // forward stepper: W[wA] = the Laplacian of the current slice
+    M_GRAD = 1u << 14,      // adjoint stepper: img += W[wImg] * n
 };
 
 // Where a window capture V goes (StepArgs::winOut).
@@ -259,6 +261,10 @@ constexpr unsigned MODE_TOMO_ADJ_CAP_WIN = M_ADJ | M_SS_SLICE | M_WIN;
 // Wavefield saving: the Born scattered field captured at the coarse rate
 // into ShotSlot::img (the source wavefield W stays readable).
 constexpr unsigned MODE_BORN_SCAT_CAP = M_SS_BORN | M_CAPTURE | M_CAP_ALT;
+// Velocity gradient: the source field with the Laplacian of each slice kept,
+// and the adjoint field imaged against it.
+constexpr unsigned MODE_SRC_LAP = M_INJ_SIG | M_LAP;
+constexpr unsigned MODE_ADJ_GRAD = MODE_NL_ADJ | M_GRAD;
 
 // spb: shots advanced per workgroup (1 or 2), sharing the tile's v2dt2 and sponge.
 // e0/e1 (optional): events timestamped by the dispatch itself.
@@ -274,7 +280,7 @@ hipError_t launch_step_generic(unsigned mode, int tz, int tx, const StepArgs& a,
                                hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // The step with four z-points per lane (wide.hip), on tiles kWideTZ x tx, for
 // grids wide_grid_ok accepts.  tx == 16: MODE_NL_FWD, MODE_NL_ADJ, MODE_SRC,
-// and with a free surface MODE_SRC_WIN, MODE_BORN_SCAT, MODE_BORN_SCAT_PRE,
+// MODE_SRC_LAP and MODE_ADJ_GRAD, and with a free surface MODE_SRC_WIN, MODE_BORN_SCAT, MODE_BORN_SCAT_PRE,
 // MODE_BORN_REC and MODE_REC_WIN too; tx == 32: MODE_SRC_WIN and
 // MODE_BORN_SCAT_PRE.
 constexpr int kWideTZ = 64, kWideTX = 16, kWidePairTX = 32;

@@ -109,6 +109,7 @@ __device__ __forceinline__ void wide_block(const StepArgs& a, const ShotSlot& S,
     f4 sA[HAS_SS ? PX : 1], sB[HAS_SS ? PX : 1], mm[SSB ? PX : 1];
     cgf* ssa = nullptr;
     cgf* ssb = nullptr;
+    f4 gw[(MODE & M_GRAD) ? PX : 1], gi[(MODE & M_GRAD) ? PX : 1];
     if constexpr (HAS_SS) {
         ssa = G(S.W) + F.wA;
         if (useB) ssb = G(S.W) + F.wB;
@@ -123,6 +124,10 @@ __device__ __forceinline__ void wide_block(const StepArgs& a, const ShotSlot& S,
             if constexpr (HAS_SS) {
                 sA[j] = ld4s(ssa, o, SSP && a.ntW);
                 if (useB) sB[j] = ld4s(ssb, o, SSP && a.ntW);
+            }
+            if constexpr (MODE & M_GRAD) {
+                gw[j] = ld4s(G(S.W) + a.wImg, o, a.ntW);
+                gi[j] = ld4(G(S.img), o);
             }
             if constexpr (SPONGE) {
                 const int dx = imin(gx + j - FAT, nx - 1 - FAT - gx - j);
@@ -158,7 +163,7 @@ __device__ __forceinline__ void wide_block(const StepArgs& a, const ShotSlot& S,
     }
 
     const bool surf = FS && z0 == 0 && zq == 0;                                 // the thread's first row is the surface
-    f4 nv[PX], cur[WIN ? PX : 1];
+    f4 nv[PX], cur[WIN ? PX : 1], lv[(MODE & M_LAP) ? PX : 1];
     if (ok) {
         f4a w[PX + 2 * FAT];
 #pragma unroll
@@ -198,6 +203,7 @@ __device__ __forceinline__ void wide_block(const StepArgs& a, const ShotSlot& S,
                     + a.xc[3] * (w[j + 8][r] + w[j + 2][r])
                     + a.xc[4] * (w[j + 9][r] + w[j + 1][r])
                     + a.xc[5] * (w[j + 10][r] + w[j + 0][r]);
+                if constexpr (MODE & M_LAP) lv[j][r] = lap;
                 const bool onSurf = FS && r == 0 && surf;
                 // forward: the old slice's surface value reads as zero, as the
                 // reference zeroed it when it was the current one
@@ -282,6 +288,8 @@ __device__ __forceinline__ void wide_block(const StepArgs& a, const ShotSlot& S,
         A = G(ADJ ? S.ss[a.ssA] : S.W) + (ADJ ? a.ssOffA : F.wA);
         B = G(ADJ ? S.ss[a.ssB] : S.W) + (ADJ ? a.ssOffB : F.wB);
     }
+    gf* lapW = (MODE & M_LAP) ? G(S.W) + F.wA : nullptr;
+    gf* gImg = (MODE & M_GRAD) ? G(S.img) : nullptr;
     gf* imgI = nullptr;
     cgf* imgW = nullptr;
     if constexpr (MODE & M_IMAGE) {
@@ -342,6 +350,8 @@ __device__ __forceinline__ void wide_block(const StepArgs& a, const ShotSlot& S,
                     }
                 }
             }
+            if constexpr (MODE & M_LAP) st4s(lapW, o, lv[j], a.ntW);
+            if constexpr (MODE & M_GRAD) st4(gImg, o, gi[j] + gw[j] * n);
             st4(F.po, o, n);
         }
     }
@@ -464,6 +474,8 @@ hipError_t launch_wide(unsigned mode, int tx, const StepArgs& a, hipStream_t s, 
         case MODE_NL_FWD: k = k_wide<kWideTZ, 1, MODE_NL_FWD, false>; break;
         case MODE_NL_ADJ: k = k_wide<kWideTZ, 1, MODE_NL_ADJ, false>; break;
         case MODE_SRC: k = k_wide<kWideTZ, 1, MODE_SRC, false>; break;
+        case MODE_SRC_LAP: k = k_wide<kWideTZ, 1, MODE_SRC_LAP, false>; break;
+        case MODE_ADJ_GRAD: k = k_wide<kWideTZ, 1, MODE_ADJ_GRAD, false>; break;
         }
     }
     if (!k) return hipErrorInvalidValue;

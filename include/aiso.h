@@ -246,7 +246,9 @@ aiso_status aiso_nl_forward_noalloc(aiso_ctx* ctx, int add, const float* model, 
  * model: the source signals of aiso_nl_forward ([nShotSig][nSrcDev][nts]);
  * dataGrad: dJ/d(data) [nShot][nRec][nts]; velGrad (out): dJ/d(velocity)
  * on the padded grid [nx][nz], overwritten.  checkpointEvery: fine steps
- * between checkpoints (0 = ceil(sqrt(ntw - 1))).  mem applies to dataGrad
+ * between checkpoints (0: as many as a quarter of the free device memory, at
+ * most 64 GB, holds slices for, at least ceil(sqrt(ntw - 1)); a gradient
+ * whose steps all fit recomputes nothing).  mem applies to dataGrad
  * and velGrad (the model is read through the host either way). */
 aiso_status aiso_nl_velocity_gradient(aiso_ctx* ctx, const float* model, int nShotSig,
                                       const float* dataGrad, float* velGrad,

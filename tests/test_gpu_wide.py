@@ -60,3 +60,20 @@ def test_modeling_of_many_shots(nzi, nxi, shots):
     ref = O.nl_forward(g, c.vel, osrc, orec, w, "f")
     assert np.abs(ref).max() > 0
     np.testing.assert_array_equal(d, ref)
+
+
+@pytest.mark.parametrize("nzi,nxi,shots,sub,every", [
+    (64, 64, 1, 2, 0), (80, 48, 2, 2, 1), (112, 80, 3, 3, 7), (64, 112, 2, 2, 39), (176, 112, 5, 1, 20)])
+def test_velocity_gradient(nzi, nxi, shots, sub, every):
+    """Against the one-point-per-lane kernels and their imaging kernel too."""
+    A, c, ctx, g, srcs, recs, osrc, orec = _setup(nzi, nxi, shots, sub, False, 40 // sub)
+    m = c.wavelet[None, None, :].copy()
+    dr = np.random.default_rng(6).standard_normal((shots, recs[0].nDev, c.nts)).astype(np.float32)
+    ref = O.nl_velocity_gradient(g, c.vel, osrc, orec, m, dr, "f")
+    assert np.abs(ref).max() > 0
+    for tile in (0, 3232):
+        if tile:
+            ctx.set_option("tileAdj", tile)
+        grad = np.zeros((c.nx, c.nz), np.float32)
+        ctx.nl_velocity_gradient(m, dr, grad, srcs, recs, checkpoint_every=every)
+        np.testing.assert_array_equal(grad, ref)
