@@ -231,6 +231,32 @@ DevGeom* dev_geom_steps(aiso_ctx* c, const aiso_device* d, int config, bool regi
     return out;
 }
 
+StepsArgs steps_args(const aiso_ctx* c, int config, const ShotSlot* slots, int nShot)
+{
+    const FdParams& p = c->p;
+    const StepsConfig& t = kStepsConfig[config];
+    StepsArgs x{};
+    x.slots = slots;
+    x.v2dt2 = c->v2dt2.as<float>();
+    x.cd = c->cd.as<float>();
+    x.nz = p.nz; x.nx = p.nx; x.minPad = p.minPad; x.nts = p.nts; x.ntw = p.ntw;
+    x.nshots = nShot;
+    x.tilesZ = (p.nz - 2 * kFat + t.tz - 1) / t.tz;
+    x.ntiles = x.tilesZ * ((p.nx - 2 * kFat + t.tx - 1) / t.tx);
+    for (int k = 0; k < 6; ++k) { x.zc[k] = p.zc[k]; x.xc[k] = p.xc[k]; }
+    return x;
+}
+
+void set_steps(const FdParams& p, StepsArgs& x, int itw, int dir)
+{
+    for (int i = 0; i < x.n; ++i, itw += dir) {
+        x.itw[i] = itw;
+        x.its[i] = itw / p.sub;
+        x.wi[i][0] = p.filt[itw % p.sub + 1];
+        x.wi[i][1] = p.filt[p.h() + itw % p.sub + 1];
+    }
+}
+
 hipEvent_t pooled_event(aiso_ctx* c)
 {
     if (!c->evPool.empty()) {
@@ -447,6 +473,25 @@ aiso_status guard(F&& f)
     }
 }
 
+// Tiles of the gradient's passes on k_steps, by their workgroups over a batch.
+// Their streams of W and the image weigh on the one-step kernels, so that the
+// largest tile beats those at any count.  Time of misfit and gradient (MI355X),
+// 32 x 32 / 64 x 32 / 64 x 64 tiles / one step per launch:
+//   1 shot of 150 x 300, 104 workgroups of 32 x 32:     6.3 /  6.9 /  8.2 /  8.0 ms
+//   4 shots of 200 x 400, 320 workgroups of 64 x 32:   12.7 / 11.3 / 13.0 / 15.9 ms
+//   4 shots of 700 x 1500, 2600 workgroups of 64 x 32: 40.8 / 31.6 / 28.1 / 33.4 ms
+//   16 shots of 500 x 1200, 3360 of 64 x 64:           65.6 / 49.7 / 42.3 / 49.8 ms
+static int grad_steps_config(const aiso_ctx* c, int nShot)
+{
+    for (int i = 0; i + 1 < kStepsConfigs; ++i) {
+        const StepsConfig& t = kStepsConfig[i];
+        if ((long)((c->p.nz - 2 * kFat + t.tz - 1) / t.tz) * ((c->p.nx - 2 * kFat + t.tx - 1) / t.tx) * nShot <=
+            (i == 0 ? 256 : 512))
+            return i;
+    }
+    return kStepsConfigs - 1;
+}
+
 // Velocity gradient of the nonlinear operator by the adjoint-state method
 // (no counterpart in the reference, whose FWI takes the Born adjoint as its
 // gradient, PY/fwiMain.py:123-142).  The forward recursion of one fine step,
@@ -458,11 +503,13 @@ aiso_status guard(F&& f)
 // one forward pass that writes a checkpoint (the pair of slices) at the start
 // of each segment but the last, whose L p_{t-1} it keeps in W (K slices);
 // then per segment, last first, the recompute of its forward steps into W
-// (but for the last) and its K adjoint steps, which image against W.  The
-// one-point-per-lane kernels keep p_{t-1} itself and image in a kernel of its
+// (but for the last) and its K adjoint steps, which image against W, several
+// steps per launch (k_steps) or one (k_wide).  The one-point-per-lane kernels
+// keep p_{t-1} itself and image in a kernel of its
 // own, which makes the Laplacian again; with them every segment is
 // recomputed.  Misfit and gradient of 8 shots of 400 x 1000 points, 800 samples
-// (MI355X): 132 ms with those and K = 40, 95 ms with one segment.
+// (MI355X): 132 ms with those and K = 40, 95 ms with one segment, 77 ms with
+// three steps per launch.
 void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dataGrad, float* velGrad,
                  aiso_device* const* srcs, int nShot, aiso_device* const* recs, int nRec, int every, int mem)
 {
@@ -515,6 +562,7 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
     // (k_grad), which makes the Laplacian again, takes it from slices without
     // the sources of the FAT ring.
     const bool fused = c->wide && maxSrcRing == 0;
+    const bool multi = fused && maxRecRing == 0 && p.minPad <= kStepsPadMax;   // several steps per launch
     // 16 shots per batch by default, 8 per lane: at 400 x 1000 with 8 per
     // batch a lane's launch covers the GPU about once (MI355X: 230 against
     // 254 Gpts/s for 16; 12 and 32 gave 249 and 251).
@@ -535,13 +583,14 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
     const int nSeg = (T - 1) / K + 1;                  // segments start at t = 0, K, 2K, ... < T
     const int nCk = fused ? nSeg - 1 : nSeg;           // of which these are started from checkpoints
     // per shot: forward pair, adjoint pair, K segment slices, gradient, checkpoints
-    const size_t perShot = (size_t)(2 + 2 + K + 1 + 2 * nCk) * nzx * 4 + (size_t)nRecRegMax * p.nts * 4 +
+    const size_t perShot = (size_t)((multi ? 8 : 4) + K + 1 + 2 * nCk) * nzx * 4 + (size_t)nRecRegMax * p.nts * 4 +
                            2 * (size_t)nSrcRegMax * p.ntw * 4;
     B = std::min(B, (int)std::max<size_t>(1, (size_t)(freeB * 0.85) / perShot));
     B = std::min(B, nShot);
     c->batchUsed = B;
-    float* pairs = (float*)c->pairs.need((size_t)B * 2 * nzx * 4);
-    float* pairsA = (float*)c->pairsQ.need((size_t)B * 2 * nzx * 4);
+    const int steps = multi ? grad_steps_config(c, B) : -1, nSl = steps >= 0 ? 4 : 2;   // slices per field
+    float* pairs = (float*)c->pairs.need((size_t)B * nSl * nzx * 4);
+    float* pairsA = (float*)c->pairsQ.need((size_t)B * nSl * nzx * 4);
     float* W = (float*)c->W.need((size_t)B * K * nzx * 4);
     float* img = (float*)c->img.need((size_t)B * nzx * 4);
     float* ck = nCk > 0 ? (float*)c->ck.need((size_t)B * 2 * nCk * nzx * 4) : nullptr;
@@ -581,8 +630,7 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
             DevGeom* rg = recG[nRec == 1 ? 0 : shot];
             ShotSlot& F = fs[k];
             std::memset(&F, 0, sizeof(F));
-            F.p[0] = pairs + (size_t)k * 2 * nzx;
-            F.p[1] = F.p[0] + nzx;
+            for (int i = 0; i < nSl; ++i) F.p[i] = pairs + ((size_t)k * nSl + i) * nzx;
             F.W = W + (size_t)k * K * nzx;
             F.img = img + (size_t)k * nzx;
             F.dreg = dreg + (size_t)k * nRecRegMax * p.nts;
@@ -597,9 +645,18 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
             F.nRecRing = rg->nRing;
             ShotSlot& A = as[k];
             A = F;
-            A.p[0] = pairsA + (size_t)k * 2 * nzx;
-            A.p[1] = A.p[0] + nzx;
+            for (int i = 0; i < nSl; ++i) A.p[i] = pairsA + ((size_t)k * nSl + i) * nzx;
             A.sig = sigA + (size_t)k * nSrcRegMax * p.ntw;
+            if (steps >= 0) {
+                const DevGeom *src = dev_geom_steps(c, srcs[shot], steps, true), *own = dev_geom_steps(c, srcs[shot], steps, false),
+                              *rec = dev_geom_steps(c, recs[nRec == 1 ? 0 : shot], steps, true);
+                F.srcTile = src->tilePtr.as<int>();
+                F.srcEnt = src->ent.as<int2>();
+                A.srcOwnTile = own->tilePtr.as<int>();
+                A.srcOwnEnt = own->ent.as<int2>();
+                A.recTile = rec->tilePtr.as<int>();
+                A.recEnt = rec->ent.as<int2>();
+            }
             const Geometry& sgm = srcs[shot]->g;
             const float* m = hModel.data() + (size_t)(nShotSig == 1 ? 0 : shot) * nSrcDev * p.nts;
             std::vector<float> fine = nl_source(c, sgm, m);
@@ -618,8 +675,8 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
         HIPC(hipMemcpyAsync(sig, sigHost.data(), sigHost.size() * 4, hipMemcpyHostToDevice, s));
         HIPC(launch_fill(sigA, (long)nb * nSrcRegMax * p.ntw, s));
         HIPC(launch_fill(img, (long)nb * nzx, s));
-        HIPC(launch_fill(pairs, (long)nb * 2 * nzx, s));
-        HIPC(launch_fill(pairsA, (long)nb * 2 * nzx, s));
+        HIPC(launch_fill(pairs, (long)nb * nSl * nzx, s));
+        HIPC(launch_fill(pairsA, (long)nb * nSl * nzx, s));
         // The recompute writes interior points only; the imaging kernel's
         // Laplacian reads the FAT ring of these slices, which must hold 0.
         if (!fused) HIPC(launch_fill(W, (long)nb * K * nzx, s));
@@ -639,11 +696,11 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
             }
             return s;
         };
-        auto save = [&](int j, int cur) {
+        auto save = [&](int j, int cur, int old) {
             for (int k = 0; k < nb; ++k) {
                 hipStream_t ls = lane_of(k);
                 HIPC(hipMemcpyAsync(ckSlice(k, j, 0), fs[k].p[cur], nzx * 4, hipMemcpyDeviceToDevice, ls));
-                HIPC(hipMemcpyAsync(ckSlice(k, j, 1), fs[k].p[cur ^ 1], nzx * 4, hipMemcpyDeviceToDevice, ls));
+                HIPC(hipMemcpyAsync(ckSlice(k, j, 1), fs[k].p[old], nzx * 4, hipMemcpyDeviceToDevice, ls));
             }
         };
         auto ring_lanes = [&](unsigned mode, const StepArgs& x, int mr) {
@@ -672,13 +729,52 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
         c->curLanes = std::max(1, std::min(c->lanes, nb));
         if (c->curLanes > 1) ensure_lanes(c);
         fork_lanes(c);
+        // One fine step t from slice cur, or several in one launch: x.n steps
+        // from t on (itw = t - 1), the field's current pair x.pair.
+        StepsArgs xf{}, xa{};
+        if (steps >= 0) {
+            xf = steps_args(c, steps, dF, nb);
+            xa = steps_args(c, steps, dA, nb);
+            xf.wStep = xa.wStep = nzx;
+        }
+        auto multi_steps = [&](StepsArgs& x, unsigned mode, int kind, int itw, int count, long wOff) {
+            const int dir = mode == MODE_ADJ_GRAD ? -1 : 1;
+            for (int done = 0; done < count; done += x.n) {
+                x.n = std::min(kStepsConfig[steps].k, count - done);
+                set_steps(p, x, itw + dir * done, dir);
+                x.wOff = wOff + dir * (long)done * nzx;
+                for (int l = 0; l < c->curLanes; ++l) {
+                    int k0, cnt;
+                    lane_range(nb, c->curLanes, l, k0, cnt);
+                    if (cnt == 0) continue;
+                    StepsArgs y = x;
+                    y.slots = x.slots + k0;
+                    y.nshots = cnt;
+                    hipEvent_t e0 = nullptr, e1 = nullptr;
+                    if (sample_event(c, kind)) {
+                        e0 = pooled_event(c);
+                        e1 = pooled_event(c);
+                        c->ev.push_back({e0, e1, kind, double(p.interior()) * cnt * x.n});
+                    }
+                    HIPC(launch_steps(steps, mode, y, lane_stream(c, l), e0, e1));
+                }
+                x.pair ^= 1;
+            }
+        };
         int cur = 1;
         const int tLast = (nSeg - 1) * K;              // the fused pass goes on into the last segment
-        if (nCk > 0) save(0, cur);
-        for (int t = 1; t < (fused ? tLast + 1 : T); ++t) {
-            fwd_step(t, cur, -1);
-            cur ^= 1;
-            if (t % K == 0 && t / K < nCk) save(t / K, cur);
+        if (nCk > 0) save(0, 1, 0);
+        if (steps >= 0) {
+            for (int j = 0; j < nCk; ++j) {
+                multi_steps(xf, MODE_STEPS_SRC, AISO_K_SRC, j * K, K, 0);
+                if (j + 1 < nCk) save(j + 1, 2 * xf.pair, 2 * xf.pair + 1);
+            }
+        } else {
+            for (int t = 1; t < (fused ? tLast + 1 : T); ++t) {
+                fwd_step(t, cur, -1);
+                cur ^= 1;
+                if (t % K == 0 && t / K < nCk) save(t / K, cur, cur ^ 1);
+            }
         }
         // backward, segment by segment
         StepArgs r = a;
@@ -690,11 +786,18 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
             if (j < nCk) {
                 for (int k = 0; k < nb; ++k) {
                     hipStream_t ls = lane_of(k);
-                    HIPC(hipMemcpyAsync(fs[k].p[1], ckSlice(k, j, 0), nzx * 4, hipMemcpyDeviceToDevice, ls));
-                    HIPC(hipMemcpyAsync(fs[k].p[0], ckSlice(k, j, 1), nzx * 4, hipMemcpyDeviceToDevice, ls));
+                    const int i = steps >= 0 ? 0 : 1;   // the current slice
+                    HIPC(hipMemcpyAsync(fs[k].p[i], ckSlice(k, j, 0), nzx * 4, hipMemcpyDeviceToDevice, ls));
+                    HIPC(hipMemcpyAsync(fs[k].p[i ^ 1], ckSlice(k, j, 1), nzx * 4, hipMemcpyDeviceToDevice, ls));
                     if (!fused) HIPC(hipMemcpyAsync(fs[k].W, ckSlice(k, j, 0), nzx * 4, hipMemcpyDeviceToDevice, ls));
                 }
                 cur = 1;
+                xf.pair = 0;
+            }
+            if (steps >= 0) {                            // W[t - 1 - t0] = L(p_{t-1}), p_t; then nu_t and its image
+                multi_steps(xf, MODE_SRC_LAP, AISO_K_SRC, t0, t1 - t0, 0);
+                multi_steps(xa, MODE_ADJ_GRAD, AISO_K_NL_ADJ, t1 - 1, t1 - t0, (long)(t1 - 1 - t0) * nzx);
+                continue;
             }
             if (fused) {
                 for (int t = t0 + 1; t <= t1; ++t) {     // W[t - 1 - t0] = L(p_{t-1}), p_t

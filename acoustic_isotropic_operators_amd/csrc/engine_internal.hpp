@@ -239,6 +239,9 @@ int tiles_z2(const aiso_ctx* c);
 int tiles_x2(const aiso_ctx* c);
 DevGeom* dev_geom_pair2(aiso_ctx* c, const aiso_device* d, bool region);
 DevGeom* dev_geom_steps(aiso_ctx* c, const aiso_device* d, int config, bool region);
+StepsArgs steps_args(const aiso_ctx* c, int config, const ShotSlot* slots, int nShot);
+// Samples and weights of the x.n fine steps itw, itw + dir, ...
+void set_steps(const FdParams& p, StepsArgs& x, int itw, int dir);
 
 hipEvent_t pooled_event(aiso_ctx* c);
 void wait_default_stream(aiso_ctx* c);

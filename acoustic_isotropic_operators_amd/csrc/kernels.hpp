@@ -171,10 +171,10 @@ struct Rec2Args {
 // to p[2 (pair ^ 1)], p[2 (pair ^ 1) + 1].
 constexpr int kStepsMax = 4, kStepsPadMax = 200;    // steps per launch, sponge width
 struct StepsConfig {
-    int tz, tx, k;                  // tile and steps per launch
+    int tz, tx, k, px;              // tile, steps per launch, columns per thread
 };
 constexpr int kStepsConfigs = 3;
-constexpr StepsConfig kStepsConfig[kStepsConfigs] = {{32, 32, 4}, {64, 32, 3}, {64, 64, 3}};
+constexpr StepsConfig kStepsConfig[kStepsConfigs] = {{32, 32, 4, 1}, {64, 32, 3, 1}, {64, 64, 3, 2}};
 struct StepsArgs {
     const ShotSlot* slots;
     const float* v2dt2;
@@ -186,6 +186,7 @@ struct StepsArgs {
     int its[kStepsMax];             // per step: coarse sample of the data weights wi, column of sig
     int itw[kStepsMax];
     float wi[kStepsMax][2];
+    long wOff, wStep;               // M_LAP, M_GRAD: W slice of the first step, and from slice to slice in time
 };
 constexpr int steps_slices(bool adj) { return adj ? 4 : 3; }   // slices in LDS
 constexpr int steps_up4(int x) { return (x + 3) / 4 * 4; }
@@ -290,9 +291,11 @@ hipError_t launch_wide(unsigned mode, int tx, const StepArgs& a, hipStream_t s, 
 // The lockstep Born forward's step of both fields (launch_fwd_pair), on tiles
 // kWideTZ x kWidePairTX.
 hipError_t launch_wide_pair(const StepArgs& a, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
-// Up to K fine steps of the nonlinear forward or adjoint (steps.hip), no
-// source or receiver in the FAT ring, no free surface.
-hipError_t launch_steps(int config, bool adj, const StepsArgs& a, hipStream_t s, hipEvent_t e0 = nullptr,
+// Up to K fine steps (steps.hip), no source or receiver in the FAT ring, no
+// free surface: MODE_NL_FWD, MODE_NL_ADJ, MODE_STEPS_SRC, MODE_SRC_LAP,
+// MODE_ADJ_GRAD.
+constexpr unsigned MODE_STEPS_SRC = M_INJ_SIG;
+hipError_t launch_steps(int config, unsigned mode, const StepsArgs& a, hipStream_t s, hipEvent_t e0 = nullptr,
                         hipEvent_t e1 = nullptr);
 hipError_t launch_ring(unsigned mode, const StepArgs& a, int maxRing, hipStream_t s);
 // One fine step of every window of a launch (MODE_NL_FWD).  grid: workgroups,

@@ -1255,31 +1255,17 @@ void Call::pass_steps()
     const bool adj = is_adj(q.op);
     const int kind = adj ? AISO_K_NL_ADJ : AISO_K_NL_FWD, T = p.ntw - 1;
     const StepsConfig& t = kStepsConfig[steps];
-    StepsArgs x{};
-    x.slots = dSlots;
-    x.v2dt2 = base.v2dt2;
-    x.cd = base.cd;
-    x.nz = p.nz; x.nx = p.nx; x.minPad = p.minPad; x.nts = p.nts; x.ntw = p.ntw;
-    x.nshots = nb;
-    x.tilesZ = (p.nz - 2 * kFat + t.tz - 1) / t.tz;
-    x.ntiles = x.tilesZ * ((p.nx - 2 * kFat + t.tx - 1) / t.tx);
-    for (int k = 0; k < 6; ++k) { x.zc[k] = p.zc[k]; x.xc[k] = p.xc[k]; }
+    StepsArgs x = steps_args(c, steps, dSlots, nb);
     for (int done = 0; done < T; done += x.n) {
         x.n = std::min(t.k, T - done);
-        for (int i = 0; i < x.n; ++i) {
-            const int itw = adj ? T - 1 - done - i : done + i, it2 = itw % p.sub;
-            x.itw[i] = itw;
-            x.its[i] = itw / p.sub;
-            x.wi[i][0] = f[it2 + 1];
-            x.wi[i][1] = f[h + it2 + 1];
-        }
+        set_steps(p, x, adj ? T - 1 - done : done, adj ? -1 : 1);
         hipEvent_t e0 = nullptr, e1 = nullptr;
         if (sample_event(c, kind)) {
             e0 = pooled_event(c);
             e1 = pooled_event(c);
             c->ev.push_back({e0, e1, kind, double(p.interior()) * nb * x.n});
         }
-        HIPC(launch_steps(steps, adj, x, s, e0, e1));
+        HIPC(launch_steps(steps, adj ? MODE_NL_ADJ : MODE_NL_FWD, x, s, e0, e1));
         x.pair ^= 1;
     }
     if (!adj) record_data();

@@ -52,10 +52,14 @@ __device__ __forceinline__ float injected(const StepsArgs& a, const ShotSlot& S,
     }
 }
 
-template <int TZ, int TX, int K, int NTH, int PX, bool ADJ>
+template <int TZ, int TX, int K, int NTH, int PX, unsigned MODE>
 __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
 {
     using T = StepsShape<TZ, TX, K>;
+    constexpr bool ADJ = MODE & M_ADJ, REC = MODE & (M_REC_DATA | M_REC_SIG);
+    // OWN: each thread keeps a quad of the tile's points over the steps
+    constexpr bool OWN = MODE & M_GRAD;
+    static_assert(TZ / 4 * TX <= NTH, "a thread per quad of the tile");
     constexpr int E = T::E, HZ = T::HZ, LZ = T::LZ, SZ = T::SZ;
     __shared__ __attribute__((aligned(16))) float lds[steps_slices(ADJ) * SZ + kStepsPadMax + 1];
     __shared__ int fewI[kFew];
@@ -82,7 +86,8 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
     cgf* VG = G(a.v2dt2);
     // Sparse entries: those of the region inject, those of the tile record.
     const int i0 = (ADJ ? S.recTile : S.srcTile)[tile], i1 = (ADJ ? S.recTile : S.srcTile)[tile + 1];
-    const int r0 = (ADJ ? S.srcOwnTile : S.recOwnTile)[tile], r1 = (ADJ ? S.srcOwnTile : S.recOwnTile)[tile + 1];
+    const int r0 = REC ? (ADJ ? S.srcOwnTile : S.recOwnTile)[tile] : 0;
+    const int r1 = REC ? (ADJ ? S.srcOwnTile : S.recOwnTile)[tile + 1] : 0;
     {
         cgf* C = G(S.p[2 * a.pair]);
         cgf* O = G(S.p[2 * a.pair + 1]);
@@ -114,6 +119,20 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
                     *(f4a*)&V0[li[k]] = v[k];
                 }
             }
+    }
+    // The thread's quad of the tile, and what it holds for the steps: the image
+    // and the samples of W it is made from.
+    const int oq = t % (TZ / 4), oc = t / (TZ / 4), oli = T::index(4 * oq, oc);
+    const bool own = OWN && t < TZ / 4 * TX && z0 + 4 * oq < nzi && x0 + oc < nxi;
+    const unsigned ooff = own ? at(z0 + 4 * oq, x0 + oc) : 0u;
+    f4 img = (f4)0.f, ow[OWN ? K : 1];
+    if constexpr (MODE & M_GRAD) {
+        if (own) {
+            img = ld4(G(S.img), ooff);
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (k < a.n) ow[k] = ld4s(G(S.W) + (a.wOff - k * a.wStep), ooff, 1);
+        }
     }
     // The first NTH entries of each list are held by a thread for all steps.
     const int2* ie = ADJ ? S.recEnt : S.srcEnt;
@@ -201,7 +220,7 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
                 if constexpr (ADJ) cc = *(const f4a*)&cur[li];
                 f4 d = (f4)1.f;
                 if constexpr (SPONGE.v) d = damp(z0 + row, x0 + c + j);
-                f4 n;
+                f4 n, la;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     // 10th-order Laplacian in the reference's summation order: z terms, then x terms
@@ -218,9 +237,13 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
                                     + a.xc[4] * (w[j + 9][r] + w[j + 1][r])
                                     + a.xc[5] * (w[j + 10][r] + w[j + 0][r]);
                     const float od = SPONGE.v ? o[r] * d[r] : o[r];            // second damping of the old slice
+                    if constexpr (MODE & M_LAP) la[r] = lap;
                     if constexpr (ADJ) n[r] = lap + cc[r] + cc[r] - od;
                     else n[r] = v[r] * lap + cc[r] + cc[r] - od;
                 }
+                if constexpr (MODE & M_LAP)
+                    if (LAST || (row >= 0 && row < TZ && c + j >= 0 && c + j < TX))
+                        st4s(G(S.W) + (a.wOff + i * a.wStep), at(z0 + row, x0 + c + j), la, 1);
                 for (int k = 0; k < few; ++k) {
                     const int r = fewI[k] - li;
                     if (r >= 0 && r < 4) n[r] += fewV[i][k];
@@ -233,7 +256,7 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
                         st4(Cn, off, n);
                         st4(On, off, cc);
                     }
-                    if (inj || rec) *(f4a*)&old[li] = n;
+                    if (inj || rec || OWN) *(f4a*)&old[li] = n;
                 } else {
                     *(f4a*)&old[li] = n;
                     if constexpr (ADJ)
@@ -276,8 +299,16 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
                 });
             }
         }
-        if (!LAST || rec) __syncthreads();
+        if (!LAST || rec || OWN) __syncthreads();
         const float* const n = old;
+        if constexpr (MODE & M_GRAD) {
+            if (own) {
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    if (k == i) img = img + ow[k] * *(const f4a*)&n[oli];
+            }
+        }
+        if constexpr (!REC) return;
         if (ri >= 0) {
 #pragma unroll
             for (int k = 0; k < K; ++k) rv[k] = k == i ? n[ri] : rv[k];
@@ -302,6 +333,8 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
     if (sponge) all(IC<1>{});
     else all(IC<0>{});
 
+    if constexpr (MODE & M_GRAD)
+        if (own) st4(G(S.img), ooff, img);
     if (ri >= 0) {
 #pragma unroll
         for (int k = 0; k < K; ++k) {
@@ -323,27 +356,41 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
     }
 }
 
-template <int TZ, int TX, int K, int PX>
-hipError_t launch(bool adj, const StepsArgs& a, hipStream_t s, hipEvent_t e0, hipEvent_t e1)
+template <int C, unsigned MODE>
+hipError_t launch_config(const StepsArgs& a, hipStream_t s, hipEvent_t e0, hipEvent_t e1)
 {
     constexpr int NTH = 1024;
-    auto k = adj ? k_steps<TZ, TX, K, NTH, PX, true> : k_steps<TZ, TX, K, NTH, PX, false>;
+    constexpr StepsConfig t = kStepsConfig[C];
+    auto k = k_steps<t.tz, t.tx, t.k, NTH, t.px, MODE>;
     const dim3 grid((a.ntiles * a.nshots + 7) / 8 * 8);
     if (e0 && e1) hipExtLaunchKernelGGL(k, grid, dim3(NTH), 0, s, e0, e1, 0, a);
     else hipLaunchKernelGGL(k, grid, dim3(NTH), 0, s, a);
     return hipGetLastError();
 }
 
+template <unsigned MODE>
+hipError_t launch(int config, const StepsArgs& a, hipStream_t s, hipEvent_t e0, hipEvent_t e1)
+{
+    if (config == 0) return launch_config<0, MODE>(a, s, e0, e1);
+    if (config == 1) return launch_config<1, MODE>(a, s, e0, e1);
+    return launch_config<2, MODE>(a, s, e0, e1);
+}
+
 }  // namespace
 
-hipError_t launch_steps(int config, bool adj, const StepsArgs& a, hipStream_t s, hipEvent_t e0, hipEvent_t e1)
+hipError_t launch_steps(int config, unsigned mode, const StepsArgs& a, hipStream_t s, hipEvent_t e0, hipEvent_t e1)
 {
     if (config < 0 || config >= kStepsConfigs || !wide_grid_ok(a.nz, a.nx) || a.minPad > kStepsPadMax || a.n < 1 ||
         a.n > kStepsConfig[config].k)
         return hipErrorInvalidValue;
-    if (config == 0) return launch<kStepsConfig[0].tz, kStepsConfig[0].tx, kStepsConfig[0].k, 1>(adj, a, s, e0, e1);
-    if (config == 1) return launch<kStepsConfig[1].tz, kStepsConfig[1].tx, kStepsConfig[1].k, 1>(adj, a, s, e0, e1);
-    return launch<kStepsConfig[2].tz, kStepsConfig[2].tx, kStepsConfig[2].k, 2>(adj, a, s, e0, e1);
+    switch (mode) {
+    case MODE_NL_FWD: return launch<MODE_NL_FWD>(config, a, s, e0, e1);
+    case MODE_NL_ADJ: return launch<MODE_NL_ADJ>(config, a, s, e0, e1);
+    case MODE_STEPS_SRC: return launch<MODE_STEPS_SRC>(config, a, s, e0, e1);
+    case MODE_SRC_LAP: return launch<MODE_SRC_LAP>(config, a, s, e0, e1);
+    case MODE_ADJ_GRAD: return launch<MODE_ADJ_GRAD>(config, a, s, e0, e1);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace aiso

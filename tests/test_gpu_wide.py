@@ -63,12 +63,19 @@ def test_modeling_of_many_shots(nzi, nxi, shots):
 
 
 @pytest.mark.parametrize("nzi,nxi,shots,sub,every", [
-    (64, 64, 1, 2, 0), (80, 48, 2, 2, 1), (112, 80, 3, 3, 7), (64, 112, 2, 2, 39), (176, 112, 5, 1, 20)])
+    (64, 64, 1, 2, 0), (80, 48, 2, 2, 1), (112, 80, 3, 3, 7), (64, 112, 2, 2, 39), (176, 112, 5, 1, 20),
+    (208, 240, 6, 2, 0), (208, 240, 6, 2, 11), (336, 272, 16, 2, 0), (336, 272, 16, 2, 13)])
 def test_velocity_gradient(nzi, nxi, shots, sub, every):
-    """Against the one-point-per-lane kernels and their imaging kernel too."""
+    """Several steps per launch on 32 x 32, 64 x 32 and 64 x 64 tiles, one
+    per launch where a receiver lies in the FAT ring, and the
+    one-point-per-lane kernels with their imaging kernel."""
     A, c, ctx, g, srcs, recs, osrc, orec = _setup(nzi, nxi, shots, sub, False, 40 // sub)
     m = c.wavelet[None, None, :].copy()
     dr = np.random.default_rng(6).standard_normal((shots, recs[0].nDev, c.nts)).astype(np.float32)
+    if shots == 2:
+        iz, ix = [2, 8], [9, 3]
+        recs, orec = [A.Device.ints(iz, ix, c.nz, c.nx, c.nts)], [O.Device.ints(iz, ix, c.nz, c.nx, c.nts)]
+        dr = dr[:, :2].copy()
     ref = O.nl_velocity_gradient(g, c.vel, osrc, orec, m, dr, "f")
     assert np.abs(ref).max() > 0
     for tile in (0, 3232):
