@@ -244,16 +244,22 @@ StepsArgs steps_args(const aiso_ctx* c, int config, const ShotSlot* slots, int n
     x.tilesZ = (p.nz - 2 * kFat + t.tz - 1) / t.tz;
     x.ntiles = x.tilesZ * ((p.nx - 2 * kFat + t.tx - 1) / t.tx);
     for (int k = 0; k < 6; ++k) { x.zc[k] = p.zc[k]; x.xc[k] = p.xc[k]; }
+    x.wStep = p.nzx();
+    x.ntW = c->streamNT;
     return x;
 }
 
 void set_steps(const FdParams& p, StepsArgs& x, int itw, int dir)
 {
     for (int i = 0; i < x.n; ++i, itw += dir) {
+        const int k = itw % p.sub;                  // forward it2 = k + 1, adjoint it2 = k
         x.itw[i] = itw;
         x.its[i] = itw / p.sub;
-        x.wi[i][0] = p.filt[itw % p.sub + 1];
-        x.wi[i][1] = p.filt[p.h() + itw % p.sub + 1];
+        x.first[i] = dir > 0 ? k == 0 : k == 1;
+        x.wi[i][0] = p.filt[k + 1];
+        x.wi[i][1] = p.filt[p.h() + k + 1];
+        x.fa[i] = p.filt[k];
+        x.fb[i] = p.filt[p.h() + k];
     }
 }
 
@@ -735,7 +741,6 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
         if (steps >= 0) {
             xf = steps_args(c, steps, dF, nb);
             xa = steps_args(c, steps, dA, nb);
-            xf.wStep = xa.wStep = nzx;
         }
         auto multi_steps = [&](StepsArgs& x, unsigned mode, int kind, int itw, int count, long wOff) {
             const int dir = mode == MODE_ADJ_GRAD ? -1 : 1;

@@ -187,6 +187,13 @@ struct StepsArgs {
     int itw[kStepsMax];
     float wi[kStepsMax][2];
     long wOff, wStep;               // M_LAP, M_GRAD: W slice of the first step, and from slice to slice in time
+    // Born passes: W holds coarse sample k at k * wStep.  M_WIN writes (adjoint:
+    // images against) a sample at the steps marked first, times mtil if given.
+    const float* mtil;
+    int first[kStepsMax];           // step it2 == 1 of its coarse interval
+    float fa[kStepsMax], fb[kStepsMax];
+    float wa, wb, wc;
+    int ntW;
 };
 constexpr int steps_slices(bool adj) { return adj ? 4 : 3; }   // slices in LDS
 constexpr int steps_up4(int x) { return (x + 3) / 4 * 4; }
@@ -292,8 +299,10 @@ hipError_t launch_wide(unsigned mode, int tx, const StepArgs& a, hipStream_t s, 
 // kWideTZ x kWidePairTX.
 hipError_t launch_wide_pair(const StepArgs& a, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // Up to K fine steps (steps.hip), no source or receiver in the FAT ring, no
-// free surface: MODE_NL_FWD, MODE_NL_ADJ, MODE_STEPS_SRC, MODE_SRC_LAP,
-// MODE_ADJ_GRAD.
+// free surface: MODE_NL_FWD, MODE_NL_ADJ; MODE_STEPS_SRC, MODE_SRC_LAP and
+// MODE_ADJ_GRAD of the velocity gradient; MODE_SRC, MODE_SRC_WIN (into W, times
+// mtil if given), MODE_BORN_SCAT, MODE_BORN_SCAT_PRE and MODE_REC_WIN (into the
+// image) of the Born passes.
 constexpr unsigned MODE_STEPS_SRC = M_INJ_SIG;
 hipError_t launch_steps(int config, unsigned mode, const StepsArgs& a, hipStream_t s, hipEvent_t e0 = nullptr,
                         hipEvent_t e1 = nullptr);

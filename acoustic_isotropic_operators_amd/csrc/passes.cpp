@@ -39,7 +39,8 @@ private:
     void stage_operands();
     void build_geometry();
     void plan_batches();
-    int steps_config(int shots) const;
+    int steps_config(int shots, long maxLargest) const;
+    int run_steps(int config, unsigned mode, int kind, StepsArgs x);
     void allocate();
     void prepare_model();
     void init_step_args();
@@ -49,7 +50,6 @@ private:
     void load_receiver_traces();
     void pass_pair2();
     void pass_lockstep();
-    void pass_steps();
     void pass_adjoint2();
     void pass_source();
     void passes_tomo();
@@ -81,7 +81,8 @@ private:
     int nExt = 1, nImg = 1, nRecDev = 0, nSrcDev = 0, h = 0;
     const float* f = nullptr;
     bool wemva = false, tomo = false, perShotImg = false, dataInput = false, fsurf = false, tlag = false;
-    int steps = -1;                     // k_steps configuration of the call, or -1
+    bool multi = false;                 // the call may run on k_steps
+    int stepsSrc = -1, steps = -1;      // k_steps configuration of the source and the main pass, or -1
     bool lockstep = false, pair2 = false, adj2 = false, win = false, generic = false;
     bool needW = false, needSS = false, needImg = false;
     int pairSlices = 2, ssSlices = 2, capSlices = 2, extK = 1, B = 1;
@@ -269,12 +270,15 @@ void Call::plan_batches()
     for (int i = 0; noRing && i < q.nRec; ++i) noRing = recG[i]->nRing == 0;
     pair2 = lockstep && c->pair2 && noRing && !fsurf;
     adj2 = q.op == Op::BornAdj && p.sub == 2 && c->pair2 && noRing && !fsurf;
-    // Several steps per launch (k_steps) where few workgroups carry the call.
+    // Several steps per launch (k_steps).
     const bool tileSet = is_adj(q.op) ? c->tileAdjSet : c->tileFwdSet;
-    bool multi = !is_born(q.op) && noRing && !fsurf && !tileSet && c->spb == 1 && c->occ == 6 &&
-                 p.minPad <= kStepsPadMax && wide_grid_ok(p.nz, p.nx);
-    multi = multi && steps_config(1) >= 0;
-    pairSlices = pair2 || adj2 || multi ? 4 : 2;
+    multi = (!is_born(q.op) || q.op == Op::BornFwd || q.op == Op::BornAdj) && noRing && !fsurf && !tileSet &&
+            c->spb == 1 && c->occ == 6 && p.minPad <= kStepsPadMax && wide_grid_ok(p.nz, p.nx) && !pair2 && !adj2;
+    // The lockstep kernel moves less than two passes on the largest tile: two
+    // passes take 0.87 of its time for 1 shot of 200 x 400, but 1.04 for 4 and
+    // 1.2 for 10.
+    if (multi && lockstep && steps_config(std::min(q.nShot, 32), 0) >= 0) lockstep = false;
+    pairSlices = pair2 || adj2 || (multi && !lockstep) ? 4 : 2;
     wSlices = lockstep ? 3 : p.nts;
     needW = is_born(q.op);
     needSS = is_ext(q.op) || tomo || q.op == Op::BornAdj;
@@ -331,26 +335,34 @@ void Call::plan_batches()
     B = std::min(B, q.nShot);
     B = (q.nShot + (q.nShot + B - 1) / B - 1) / ((q.nShot + B - 1) / B);   // same batch count, balanced sizes
     c->batchUsed = B;
-    steps = multi ? steps_config(B) : -1;
-    if (multi && steps < 0) {
+    // The lines for the largest tile, by its workgroups: microseconds per step,
+    // or time of the call, with it and in one-step launches.
+    //   nonlinear     320: 6.3 / 7.8   400: 7.3 / 7.8
+    //   its adjoint   240: 4.1 / 7.0   504: 8.4 / 7.4
+    //   Born, sub 3, 4: 240: 0.73 of the time, 400: 0.97, 504: 0.86
+    //   its adjoint's receiver pass, which moves the image once per launch:
+    //     640: 0.82, 840: 0.90, 1680: 0.95, 2952: 0.98, 4200: 1.03
+    if (multi && !lockstep) {
+        if (is_born(q.op)) stepsSrc = steps_config(B, 512);
+        if (q.op != Op::BornAdj) steps = steps_config(B, q.op == Op::NlAdj ? 256 : 512);
+        else if (win && c->batchRec == 0) steps = steps_config(B, 3000);
+    }
+    if (pairSlices == 4 && !pair2 && !adj2 && steps < 0 && stepsSrc < 0) {
         pairSlices = 2;
         c->bytesPerShot -= 2 * nzx * 4;
     }
 }
 
-// The tiles and steps per launch with which `shots` shots run on k_steps: the
-// smallest tile whose workgroups all run at once, one per CU, or for the
-// forward two rounds of the largest; -1: none, and the one-step kernels are
-// faster.  Microseconds per step with the largest tile and in one-step
-// launches: 304 x 512 points, 8 shots, 320 workgroups: forward 6.3 against
-// 7.8; 608 x 1312, 2 shots, 400 workgroups: forward 7.3 against 7.8; 400 x
-// 768, 6 shots, 504 workgroups: adjoint 8.4 against 7.4.
-int Call::steps_config(int shots) const
+// The tiles and steps per launch with which a pass over `shots` shots runs on
+// k_steps: the smallest tile whose workgroups all run at once, one per CU, or
+// the largest with up to maxLargest workgroups; -1: none, and the one-step
+// kernels are faster.
+int Call::steps_config(int shots, long maxLargest) const
 {
     for (int i = 0; i < kStepsConfigs; ++i) {
         const StepsConfig& t = kStepsConfig[i];
         const long n = (long)((p.nz - 2 * kFat + t.tz - 1) / t.tz) * ((p.nx - 2 * kFat + t.tx - 1) / t.tx) * shots;
-        if (n <= (i + 1 < kStepsConfigs || is_adj(q.op) ? 256 : 512)) return i;
+        if (n <= (i + 1 < kStepsConfigs ? 256 : maxLargest)) return i;
     }
     return -1;
 }
@@ -534,7 +546,7 @@ void Call::begin_batch(int first, int count)
     a = base;
     a.nshots = nb;
     a.gridLogical = a.ntiles * nb;
-    c->curLanes = pair2 || adj2 || steps >= 0 ? 1 : std::max(1, std::min(c->lanes, nb));
+    c->curLanes = pair2 || adj2 ? 1 : std::max(1, std::min(c->lanes, nb));
     if (c->curLanes > 1) ensure_lanes(c);
 }
 
@@ -586,22 +598,20 @@ void Call::upload_tables()
     if (tomo) bytes += 2 * stage_size(tb);
     if (q.op == Op::WemvaFwd) bytes += 2 * stage_size(tb);
     if (sigUp) bytes += stage_size(sigHost.size() * 4);
-    if (steps >= 0) {
-        for (int k = 0; k < nb; ++k) {
-            const aiso_device *src = q.src[b0 + k], *rec = rec_dev(b0 + k);
-            auto set = [&](const aiso_device* d, bool region, const int*& ptr, const int2*& ent) {
-                DevGeom* g = dev_geom_steps(c, d, steps, region);
-                ptr = g->tilePtr.as<int>();
-                ent = g->ent.as<int2>();
-            };
-            if (is_adj(q.op)) {
-                set(rec, true, slots[k].recTile, slots[k].recEnt);
-                set(src, false, slots[k].srcOwnTile, slots[k].srcOwnEnt);
-            } else {
-                set(src, true, slots[k].srcTile, slots[k].srcEnt);
-                set(rec, false, slots[k].recOwnTile, slots[k].recOwnEnt);
-            }
-        }
+    for (int k = 0; k < nb && (steps >= 0 || stepsSrc >= 0); ++k) {
+        const aiso_device *src = q.src[b0 + k], *rec = rec_dev(b0 + k);
+        auto set = [&](int config, const aiso_device* d, bool region, const int*& ptr, const int2*& ent) {
+            DevGeom* g = dev_geom_steps(c, d, config, region);
+            ptr = g->tilePtr.as<int>();
+            ent = g->ent.as<int2>();
+        };
+        ShotSlot& S = slots[k];
+        if (stepsSrc >= 0) set(stepsSrc, src, true, S.srcTile, S.srcEnt);
+        else if (q.op == Op::NlFwd) set(steps, src, true, S.srcTile, S.srcEnt);
+        if (steps < 0) continue;
+        if (is_adj(q.op)) set(steps, rec, true, S.recTile, S.recEnt);
+        else set(steps, rec, false, S.recOwnTile, S.recOwnEnt);
+        if (q.op == Op::NlAdj) set(steps, src, false, S.srcOwnTile, S.srcOwnEnt);
     }
     stage_begin(c, bytes);
     stage_copy(c, dSlots, slots.data(), tb);
@@ -894,7 +904,7 @@ void Call::pass_adjoint2()
 // holds the secondary source m~ * W instead.
 void Call::pass_source()
 {
-    HIPC(launch_fill(pairs, (long)nb * 2 * nzx, s));
+    HIPC(launch_fill(pairs, (long)nb * pairSlices * nzx, s));
     a.cur = 1;
     const unsigned mode = win ? MODE_SRC_WIN : MODE_SRC;
     const int winOut = q.op == Op::BornFwd ? WIN_SS : WIN_W;
@@ -902,27 +912,34 @@ void Call::pass_source()
     a.wa = f[h + 1];
     a.wb = f[h + 2 < 2 * h ? h + 2 : h + 1];
     a.wc = f[1];
-    hipEvent_t passT = pass_timer_begin(c);
-    fork_lanes(c);
-    for (int its = 0; its < p.nts - 1; ++its)
-        for (int it2 = 1; it2 <= p.sub; ++it2) {
-            a.its = its;
-            a.itwInj = its * p.sub + it2 - 1;
-            a.wA = (long)its * nzx;
-            a.wB = (long)(its + 1) * nzx;
-            a.fe = f[it2];
-            a.ff = f[h + it2];
-            a.skipA = a.fe == 0.f;
-            a.skipB = a.ff == 0.f;
-            a.assignA = its == 0 && it2 == 1;
-            a.assignB = it2 == 1;
-            a.win = it2 == 1;
-            launch_timed(c, mode, AISO_K_SRC, a, generic);
-            ring(mode, a);
-            a.cur ^= 1;
-        }
-    join_lanes(c);
-    pass_timer_end(c, passT, AISO_K_SRC, double(p.interior()) * nb * (p.ntw - 1), p.ntw - 1);
+    if (stepsSrc >= 0) {
+        StepsArgs x = steps_args(c, stepsSrc, dSlots, nb);
+        x.wa = a.wa; x.wb = a.wb; x.wc = a.wc;
+        x.mtil = winOut == WIN_SS ? mtil : nullptr;
+        a.cur = 2 * run_steps(stepsSrc, mode, AISO_K_SRC, x);
+    } else {
+        hipEvent_t passT = pass_timer_begin(c);
+        fork_lanes(c);
+        for (int its = 0; its < p.nts - 1; ++its)
+            for (int it2 = 1; it2 <= p.sub; ++it2) {
+                a.its = its;
+                a.itwInj = its * p.sub + it2 - 1;
+                a.wA = (long)its * nzx;
+                a.wB = (long)(its + 1) * nzx;
+                a.fe = f[it2];
+                a.ff = f[h + it2];
+                a.skipA = a.fe == 0.f;
+                a.skipB = a.ff == 0.f;
+                a.assignA = its == 0 && it2 == 1;
+                a.assignB = it2 == 1;
+                a.win = it2 == 1;
+                launch_timed(c, mode, AISO_K_SRC, a, generic);
+                ring(mode, a);
+                a.cur ^= 1;
+            }
+        join_lanes(c);
+        pass_timer_end(c, passT, AISO_K_SRC, double(p.interior()) * nb * (p.ntw - 1), p.ntw - 1);
+    }
     if (win)   // W[nts-1] = p(last-1)*f[h+1] + p(last)*f[h+2]
         HIPC(launch_win_tail(dSlots, nb, a.cur, winOut, f[h + 1], f[h + 2], (long)(p.nts - 1) * nzx, 0, 0, mtil,
                              p.nz, p.nx, s));
@@ -1248,40 +1265,60 @@ void Call::passes_tomo()
     }
 }
 
-// The nonlinear propagation, forward or adjoint, several fine steps per launch.
-void Call::pass_steps()
+// The fine steps of a pass, several per launch; returns the pair of slices
+// that holds the last two.
+int Call::run_steps(int config, unsigned mode, int kind, StepsArgs x)
 {
-    HIPC(launch_fill(pairs, (long)nb * 4 * nzx, s));
-    const bool adj = is_adj(q.op);
-    const int kind = adj ? AISO_K_NL_ADJ : AISO_K_NL_FWD, T = p.ntw - 1;
-    const StepsConfig& t = kStepsConfig[steps];
-    StepsArgs x = steps_args(c, steps, dSlots, nb);
+    const int T = p.ntw - 1;
+    const bool adj = mode & M_ADJ;
+    // One stream where the workgroups of all shots fit two rounds: the lanes'
+    // launches would only cost the host.
+    const int lanes = (long)x.ntiles * nb > 512 ? c->curLanes : 1;
+    hipEvent_t passT = lanes > 1 ? pass_timer_begin(c) : nullptr;
+    if (lanes > 1) fork_lanes(c);
     for (int done = 0; done < T; done += x.n) {
-        x.n = std::min(t.k, T - done);
+        x.n = std::min(kStepsConfig[config].k, T - done);
         set_steps(p, x, adj ? T - 1 - done : done, adj ? -1 : 1);
-        hipEvent_t e0 = nullptr, e1 = nullptr;
-        if (sample_event(c, kind)) {
-            e0 = pooled_event(c);
-            e1 = pooled_event(c);
-            c->ev.push_back({e0, e1, kind, double(p.interior()) * nb * x.n});
+        for (int l = 0; l < lanes; ++l) {
+            int k0, cnt;
+            lane_range(nb, lanes, l, k0, cnt);
+            if (cnt == 0) continue;
+            StepsArgs y = x;
+            y.slots = x.slots + k0;
+            y.nshots = cnt;
+            hipEvent_t e0 = nullptr, e1 = nullptr;
+            if (lanes == 1 && sample_event(c, kind)) {
+                e0 = pooled_event(c);
+                e1 = pooled_event(c);
+                c->ev.push_back({e0, e1, kind, double(p.interior()) * nb * x.n});
+            }
+            HIPC(launch_steps(config, mode, y, lanes > 1 ? lane_stream(c, l) : s, e0, e1));
         }
-        HIPC(launch_steps(steps, adj ? MODE_NL_ADJ : MODE_NL_FWD, x, s, e0, e1));
         x.pair ^= 1;
     }
-    if (!adj) record_data();
+    if (lanes > 1) join_lanes(c);
+    pass_timer_end(c, passT, kind, double(p.interior()) * nb * T, T);
+    return x.pair;
 }
 
 // Second pass of the forward operators: the nonlinear propagation, or the
 // Born / extended-Born scattered field, with the data recorded.
 void Call::pass_forward()
 {
-    HIPC(launch_fill(pairs, (long)nb * 2 * nzx, s));
+    HIPC(launch_fill(pairs, (long)nb * pairSlices * nzx, s));
     a.cur = 1;
     a.assignA = a.assignB = a.skipA = a.skipB = 0;
     unsigned mode = MODE_NL_FWD;
     int kind = AISO_K_NL_FWD;
     if (q.op == Op::BornFwd) { mode = win ? MODE_BORN_SCAT_PRE : MODE_BORN_SCAT; kind = AISO_K_BORN_SCAT; }
     if (q.op == Op::ExtFwd) { mode = MODE_EXT_SCAT; kind = AISO_K_EXT_SCAT; }
+    if (steps >= 0) {
+        StepsArgs x = steps_args(c, steps, dSlots, nb);
+        x.mtil = mtil;
+        run_steps(steps, mode, kind, x);
+        record_data();
+        return;
+    }
     int L = 0, R = 1;
     // Secondary sources of the offset-extended forward, extK samples per
     // launch into the ring, ahead of their use.
@@ -1347,7 +1384,7 @@ void Call::pass_forward()
 // (F/src/BornShotsGpuFunctions.cu:893-945).
 void Call::pass_adjoint()
 {
-    HIPC(launch_fill(pairs, (long)nb * 2 * nzx, s));
+    HIPC(launch_fill(pairs, (long)nb * pairSlices * nzx, s));
     a.cur = 1;
     a.assignA = a.assignB = a.skipA = a.skipB = 0;
     unsigned mode = MODE_NL_ADJ;
@@ -1360,6 +1397,16 @@ void Call::pass_adjoint()
     a.wa = f[1];
     a.wb = f[0];
     a.wc = f[h + 1];
+    if (steps >= 0) {
+        StepsArgs x = steps_args(c, steps, dSlots, nb);
+        x.wa = a.wa; x.wb = a.wb; x.wc = a.wc;
+        const int cur = 2 * run_steps(steps, mode, kind, x);
+        if (q.op == Op::BornAdj) {
+            HIPC(launch_win_tail(dSlots, nb, cur, WIN_IMG, f[1], f[0], 0, 0, 0, nullptr, p.nz, p.nx, s));
+            HIPC(launch_born_adj_finish(dSlots, nb, -1, base.v2dt2, c->refl.as<float>(), p.nz, p.nx, s));
+        }
+        return;
+    }
     // The stored source wavefield lets the receiver pass run the batch in
     // smaller groups, whose per-shot slices (pair + image) stay in the
     // on-die cache.
@@ -1698,8 +1745,7 @@ void Call::run()
         if (is_born(q.op) && !lockstep && !adj2) pass_source();
         if (tomo) passes_tomo();
         if (!lockstep && !adj2 && !tomo) {
-            if (steps >= 0) pass_steps();
-            else if (q.op == Op::NlFwd || q.op == Op::BornFwd || q.op == Op::ExtFwd) pass_forward();
+            if (q.op == Op::NlFwd || q.op == Op::BornFwd || q.op == Op::ExtFwd) pass_forward();
             else pass_adjoint();
         }
         reduce_images();

@@ -1,4 +1,5 @@
-// steps.hip -- several fine time steps of the nonlinear passes per launch.
+// steps.hip -- several fine time steps of a pass per launch: the nonlinear and
+// Born passes and those of the velocity gradient.
 //
 // Passes over few points are bound by launches: a one-step launch takes the
 // host 3.9 us to submit and the GPU 4.1 us for 304 x 512 points, most of it
@@ -22,7 +23,10 @@
 // workgroups all run at once (one per CU) is best: 3 shots on 32 x 32 tiles
 // take 3.75 us, 1 shot on 64 x 64 tiles 3.22.  Over many workgroups the
 // one-step kernels, which are bound by memory and not by latency, are faster
-// (16 shots of 608 x 1312 points: 411 Gpts/s against 371).
+// (16 shots of 608 x 1312 points: 411 Gpts/s against 371), but for the passes
+// that also move an image or a slice of W at every step: here they move once
+// per launch, held by one thread per quad of the tile (gradient of 8 shots of
+// 512 x 1104 points: 37 us per step of both fields, one-step launches 49).
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -58,7 +62,9 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
     using T = StepsShape<TZ, TX, K>;
     constexpr bool ADJ = MODE & M_ADJ, REC = MODE & (M_REC_DATA | M_REC_SIG);
     // OWN: each thread keeps a quad of the tile's points over the steps
-    constexpr bool OWN = MODE & M_GRAD;
+    constexpr bool WIN = MODE & M_WIN, CAP = MODE & M_CAPTURE, OWN = (MODE & M_GRAD) || WIN || CAP;
+    constexpr bool SSB = MODE & M_SS_BORN, SSP = MODE & M_SS_PRE;
+    constexpr bool INJ = MODE & (M_INJ_SIG | M_INJ_DATA);
     static_assert(TZ / 4 * TX <= NTH, "a thread per quad of the tile");
     constexpr int E = T::E, HZ = T::HZ, LZ = T::LZ, SZ = T::SZ;
     __shared__ __attribute__((aligned(16))) float lds[steps_slices(ADJ) * SZ + kStepsPadMax + 1];
@@ -85,7 +91,8 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
     gf* On = G(S.p[2 * (a.pair ^ 1) + 1]);
     cgf* VG = G(a.v2dt2);
     // Sparse entries: those of the region inject, those of the tile record.
-    const int i0 = (ADJ ? S.recTile : S.srcTile)[tile], i1 = (ADJ ? S.recTile : S.srcTile)[tile + 1];
+    const int i0 = INJ ? (ADJ ? S.recTile : S.srcTile)[tile] : 0;
+    const int i1 = INJ ? (ADJ ? S.recTile : S.srcTile)[tile + 1] : 0;
     const int r0 = REC ? (ADJ ? S.srcOwnTile : S.recOwnTile)[tile] : 0;
     const int r1 = REC ? (ADJ ? S.srcOwnTile : S.recOwnTile)[tile + 1] : 0;
     {
@@ -120,18 +127,30 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
                 }
             }
     }
-    // The thread's quad of the tile, and what it holds for the steps: the image
-    // and the samples of W it is made from.
+    // The thread's quad of the tile, and what it holds over the steps: the image
+    // and the samples of W it is made from; the quad's old and current values
+    // for the window capture; the two samples of W that a capture adds to.
     const int oq = t % (TZ / 4), oc = t / (TZ / 4), oli = T::index(4 * oq, oc);
     const bool own = OWN && t < TZ / 4 * TX && z0 + 4 * oq < nzi && x0 + oc < nxi;
     const unsigned ooff = own ? at(z0 + 4 * oq, x0 + oc) : 0u;
-    f4 img = (f4)0.f, ow[OWN ? K : 1];
-    if constexpr (MODE & M_GRAD) {
-        if (own) {
+    constexpr bool IMG = (MODE & M_GRAD) || (WIN && ADJ);
+    constexpr int NW = (MODE & M_GRAD) ? K : (K + 1) / 2;                       // windows: every other step at most
+    f4 img = (f4)0.f, ow[IMG ? NW : 1], mt = (f4)1.f, ro, rc, cA, cB;
+    if (own) {
+        if constexpr (IMG) {
             img = ld4(G(S.img), ooff);
 #pragma unroll
-            for (int k = 0; k < K; ++k)
-                if (k < a.n) ow[k] = ld4s(G(S.W) + (a.wOff - k * a.wStep), ooff, 1);
+            for (int k = 0; k < K; ++k) {
+                if (k >= a.n) continue;
+                if constexpr (MODE & M_GRAD) ow[k] = ld4s(G(S.W) + (a.wOff - k * a.wStep), ooff, a.ntW);
+                else if (a.first[k]) ow[k / 2] = ld4s(G(S.W) + (a.its[k] + 1) * a.wStep, ooff, a.ntW);
+            }
+        }
+        if constexpr (WIN && !ADJ)
+            if (a.mtil) mt = ld4(G(a.mtil), ooff);
+        if constexpr (CAP) {
+            if (!a.first[0] || a.its[0] > 0) cA = ld4(G(S.W) + a.its[0] * a.wStep, ooff);
+            if (!a.first[0]) cB = ld4(G(S.W) + (a.its[0] + 1) * a.wStep, ooff);
         }
     }
     // The first NTH entries of each list are held by a thread for all steps.
@@ -171,6 +190,12 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
             if (j <= last) acc[j] = rd[ADJ ? -j : j];
     }
     __syncthreads();
+    if constexpr (WIN) {
+        if (own) {
+            rc = *(const f4a*)&(odd ? P1 : P0)[oli];
+            ro = *(const f4a*)&(odd ? P0 : P1)[oli];
+        }
+    }
     const bool sponge = z0 - HZ < a.minPad || x0 - E < a.minPad || z0 + TZ + HZ > nzi - a.minPad || x0 + TX + E > nxi - a.minPad;
 
     auto step = [&](auto KS, auto SPONGE) {
@@ -210,6 +235,18 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
                 if (x0 + c + j < 0 || x0 + c + j >= nxi) continue;
                 const float* sj = s + j * LZ;
                 const int li = T::index(row, c + j);
+                f4 sA, sB;                                                      // secondary source
+                if constexpr (SSB || SSP) {
+                    const unsigned off = at(z0 + row, x0 + c + j);
+                    cgf* W = G(S.W) + a.its[i] * a.wStep;
+                    sA = ld4(W, off);
+                    if (a.fb[i] != 0.f) sB = ld4(W + a.wStep, off);
+                    if constexpr (SSB) {
+                        const f4 m = ld4(G(a.mtil), off);
+                        sA = m * sA;
+                        if (a.fb[i] != 0.f) sB = m * sB;
+                    }
+                }
                 const f4a up = *(const f4a*)(sj - 4), dn = *(const f4a*)(sj + 4), m = w[j + FAT];
                 const float z[14] = {sj[-5], up[0], up[1], up[2], up[3], m[0], m[1], m[2], m[3], dn[0], dn[1], dn[2], dn[3], sj[8]};
                 f4 o = *(const f4a*)&old[li];
@@ -241,9 +278,13 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
                     if constexpr (ADJ) n[r] = lap + cc[r] + cc[r] - od;
                     else n[r] = v[r] * lap + cc[r] + cc[r] - od;
                 }
+                if constexpr (SSB || SSP) {
+                    if (a.fb[i] != 0.f) n += sA * a.fa[i] + sB * a.fb[i];
+                    else n += sA * a.fa[i];
+                }
                 if constexpr (MODE & M_LAP)
                     if (LAST || (row >= 0 && row < TZ && c + j >= 0 && c + j < TX))
-                        st4s(G(S.W) + (a.wOff + i * a.wStep), at(z0 + row, x0 + c + j), la, 1);
+                        st4s(G(S.W) + (a.wOff + i * a.wStep), at(z0 + row, x0 + c + j), la, a.ntW);
                 for (int k = 0; k < few; ++k) {
                     const int r = fewI[k] - li;
                     if (r >= 0 && r < 4) n[r] += fewV[i][k];
@@ -308,6 +349,43 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
                     if (k == i) img = img + ow[k] * *(const f4a*)&n[oli];
             }
         }
+        if constexpr (WIN) {
+            if (own) {
+                const f4 nq = *(const f4a*)&n[oli];
+                if (a.first[i]) {
+                    // coarse sample from three consecutive fine slices, in the
+                    // reference's order (old, current, new)
+                    f4 v = (ro * a.wa + rc * a.wb) + nq * a.wc;
+                    if constexpr (ADJ) {
+#pragma unroll
+                        for (int k = 0; k < NW; ++k)
+                            if (k == i / 2) img = img + ow[k] * v;
+                    } else {
+                        if (a.mtil) v = mt * v;
+                        st4s(G(S.W) + a.its[i] * a.wStep, ooff, v, a.ntW);
+                    }
+                }
+                ro = rc;
+                rc = nq;
+            }
+        }
+        if constexpr (CAP) {
+            if (own) {
+                const f4 nq = *(const f4a*)&n[oli];
+                const bool first = a.first[i];                                  // of its coarse interval
+                if (first && i > 0) {
+                    st4(G(S.W) + (a.its[i] - 1) * a.wStep, ooff, cA);
+                    cA = cB;
+                }
+                // a zero weight leaves the sample as it is; a first touch
+                // writes instead of adding to a zeroed one
+                const float fe = a.wi[i][0], ff = a.wi[i][1];
+                if (fe != 0.f) cA = first && a.its[i] == 0 ? nq * fe : cA + nq * fe;
+                else if (first && a.its[i] == 0) cA = (f4)0.f;
+                if (ff != 0.f) cB = first ? nq * ff : cB + nq * ff;
+                else if (first) cB = (f4)0.f;
+            }
+        }
         if constexpr (!REC) return;
         if (ri >= 0) {
 #pragma unroll
@@ -333,8 +411,13 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
     if (sponge) all(IC<1>{});
     else all(IC<0>{});
 
-    if constexpr (MODE & M_GRAD)
-        if (own) st4(G(S.img), ooff, img);
+    if (own) {
+        if constexpr (IMG) st4(G(S.img), ooff, img);
+        if constexpr (CAP) {
+            st4(G(S.W) + a.its[a.n - 1] * a.wStep, ooff, cA);
+            st4(G(S.W) + (a.its[a.n - 1] + 1) * a.wStep, ooff, cB);
+        }
+    }
     if (ri >= 0) {
 #pragma unroll
         for (int k = 0; k < K; ++k) {
@@ -386,6 +469,11 @@ hipError_t launch_steps(int config, unsigned mode, const StepsArgs& a, hipStream
     switch (mode) {
     case MODE_NL_FWD: return launch<MODE_NL_FWD>(config, a, s, e0, e1);
     case MODE_NL_ADJ: return launch<MODE_NL_ADJ>(config, a, s, e0, e1);
+    case MODE_SRC: return launch<MODE_SRC>(config, a, s, e0, e1);
+    case MODE_SRC_WIN: return launch<MODE_SRC_WIN>(config, a, s, e0, e1);
+    case MODE_BORN_SCAT: return launch<MODE_BORN_SCAT>(config, a, s, e0, e1);
+    case MODE_BORN_SCAT_PRE: return launch<MODE_BORN_SCAT_PRE>(config, a, s, e0, e1);
+    case MODE_REC_WIN: return launch<MODE_REC_WIN>(config, a, s, e0, e1);
     case MODE_STEPS_SRC: return launch<MODE_STEPS_SRC>(config, a, s, e0, e1);
     case MODE_SRC_LAP: return launch<MODE_SRC_LAP>(config, a, s, e0, e1);
     case MODE_ADJ_GRAD: return launch<MODE_ADJ_GRAD>(config, a, s, e0, e1);

@@ -1,5 +1,4 @@
-"""The kernels that take several fine steps of a nonlinear pass per launch give
-the float oracle's results bit for bit: interior sizes that leave remainders
+"""The kernels that take several fine steps of a pass per launch give oracle's results bit for bit: interior sizes that leave remainders
 of their 32 x 32, 64 x 32 and 64 x 64 tiles, step counts that are no multiple
 of the steps per launch, sources and receivers on both sides of tile edges
 and inside a neighbour's halo, sponges narrower and wider than a tile, more
@@ -15,14 +14,13 @@ pytestmark = pytest.mark.gpu
 FAT = 5
 
 
-def _check(nzi, nxi, shots, sub, nts, pad, points):
+def _setup(nzi, nxi, shots, sub, nts, pad, points):
     from acoustic_isotropic_operators_amd import _capi as A
     c = make_case(seed=nzi * 7 + nxi, nz=nzi + 2 * FAT, nx=nxi + 2 * FAT, nShot=shots, nts=nts, sub=sub, pad=pad,
                   dts=0.001 * sub)
     ctx = A.Context(dict(nz=c.nz, nx=c.nx, dz=c.dz, dx=c.dx, nts=c.nts, dts=c.dts, sub=c.sub, alphaCos=c.alpha,
                          fMax=20.0, zPadMinus=pad, zPadPlus=pad, xPadMinus=pad, xPadPlus=pad))
     ctx.set_velocity(c.vel)
-    g = c.grid
     rng = np.random.default_rng(9)
     # sources next to tile edges, receivers as asked for
     at = [(FAT + min(nzi - 1, 31 + s % 3), FAT + (s * 31 + 30) % nxi) for s in range(shots)]
@@ -36,8 +34,14 @@ def _check(nzi, nxi, shots, sub, nts, pad, points):
     srcs = [A.Device.ints([z], [x], *dims) for z, x in at]
     osrc = [O.Device.ints([z], [x], *dims) for z, x in at]
     recs, orec = [A.Device.ints(iz, ix, *dims)], [O.Device.ints(iz, ix, *dims)]
+    return c, ctx, rng, srcs, recs, osrc, orec
+
+
+def _check(nzi, nxi, shots, sub, nts, pad, points):
+    c, ctx, rng, srcs, recs, osrc, orec = _setup(nzi, nxi, shots, sub, nts, pad, points)
+    g = c.grid
     w = rng.standard_normal((shots, 1, nts)).astype(np.float32)
-    d = np.zeros((shots, len(iz), nts), np.float32)
+    d = np.zeros((shots, recs[0].nDev, nts), np.float32)
     ctx.nl_forward(w, d, srcs, recs)
     ref = O.nl_forward(g, c.vel, osrc, orec, w, "f")
     assert np.abs(ref).max() > 0
@@ -65,3 +69,31 @@ def test_nonlinear_passes(nzi, nxi, shots, sub, nts, pad):
 def test_more_receivers_than_threads():
     _check(64, 64, 1, 2, 9, 10, "all")
     _check(64, 64, 60, 2, 5, 10, "all")
+
+
+@pytest.mark.parametrize("nzi,nxi,shots,sub,nts,pad", [
+    (32, 32, 1, 2, 2, 10),
+    (48, 80, 1, 4, 12, 10),
+    (64, 96, 2, 3, 18, 4),
+    (112, 80, 1, 1, 40, 40),
+    (208, 240, 6, 2, 20, 10),
+    (208, 240, 6, 3, 14, 10),
+    (208, 240, 14, 2, 21, 10),
+    (208, 240, 14, 4, 11, 10),
+    (208, 256, 26, 2, 14, 50),
+    (272, 304, 24, 2, 12, 10),
+])
+def test_born_passes(nzi, nxi, shots, sub, nts, pad):
+    c, ctx, rng, srcs, recs, osrc, orec = _setup(nzi, nxi, shots, sub, nts, pad, 37)
+    g = c.grid
+    wav = rng.standard_normal((1, nts)).astype(np.float32)
+    m = rng.standard_normal((c.nx, c.nz)).astype(np.float32)
+    d = np.zeros((shots, recs[0].nDev, nts), np.float32)
+    ctx.born_forward(m, d, srcs, wav, recs)
+    ref = O.born_forward(g, c.vel, osrc, [wav], orec, m, "f")
+    assert np.abs(ref).max() > 0
+    np.testing.assert_array_equal(d, ref)
+    dr = rng.standard_normal(d.shape).astype(np.float32)
+    img = np.zeros((c.nx, c.nz), np.float32)
+    ctx.born_adjoint(img, dr, srcs, wav, recs)
+    np.testing.assert_array_equal(img, O.born_adjoint(g, c.vel, osrc, [wav], orec, dr, "f"))
