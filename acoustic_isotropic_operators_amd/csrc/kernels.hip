@@ -21,6 +21,8 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device_common.hpp"
 
 namespace aiso {
@@ -1929,7 +1931,7 @@ __global__ void k_ext_adj_finish(const ShotSlot* slots, const float* __restrict_
 // imagingTimeFwdGpu (F/src/kernelsGpu.cu:337-350, lagDir = +1) and
 // imagingTimeTomoAdjGpu (:445-458, lagDir = -1) for nk samples:
 // ss_j = sum over e in [lo_j, hi_j), ascending, of mext[e] * W[k_j - lagDir * 2 (e - hExt)].
-__global__ void k_time_ss(ExtBatchArgs a)
+__global__ void k_time_ss(TimeBatchArgs a)
 {
     const ShotSlot& S = a.slots[blockIdx.y];
     const long nz = a.nz, nzx = nz * a.nx;
@@ -1940,25 +1942,25 @@ __global__ void k_time_ss(ExtBatchArgs a)
     cgf* W = G(S.W) + i;
     cgf* M = G(a.mext) + i;
     gf* SS = G(S.ss[0]) + i;
-    float acc[kExtBatchMax];
+    float acc[kTimeBatchMax];
 #pragma unroll
-    for (int j = 0; j < kExtBatchMax; ++j) acc[j] = 0.f;
+    for (int j = 0; j < kTimeBatchMax; ++j) acc[j] = 0.f;
     for (int e = a.eLo; e < a.eHi; ++e) {
         const float mv = M[nzx * e];
         const long sh = 2L * a.lagDir * (e - a.hExt) * nzx;
 #pragma unroll
-        for (int j = 0; j < kExtBatchMax; ++j)
+        for (int j = 0; j < kTimeBatchMax; ++j)
             if (j < a.nk && e >= a.lo[j] && e < a.hi[j]) acc[j] += mv * W[a.wOff[j] - sh];
     }
 #pragma unroll
-    for (int j = 0; j < kExtBatchMax; ++j)
+    for (int j = 0; j < kTimeBatchMax; ++j)
         if (j < a.nk) SS[a.ssOff[j]] = acc[j];
 }
 
 // imagingTimeAdjGpu (F/src/kernelsGpu.cu:352-364, lagDir = +1) and
 // imagingWemvaTimeAdjGpu (:366-378, lagDir = -1) for nk samples, in batch
 // order: img[e] += ss_j * W[k_j - lagDir * 2 (e - hExt)] for e in [lo_j, hi_j).
-__global__ void k_time_img(ExtBatchArgs a)
+__global__ void k_time_img(TimeBatchArgs a)
 {
     const ShotSlot& S = a.slots[blockIdx.y];
     const long nz = a.nz, nzx = nz * a.nx;
@@ -1969,40 +1971,47 @@ __global__ void k_time_img(ExtBatchArgs a)
     cgf* W = G(S.W) + i;
     cgf* SS = G(S.ss[0]) + i;
     gf* IMG = G(S.img) + i;
-    float sv[kExtBatchMax];
+    float sv[kTimeBatchMax];
 #pragma unroll
-    for (int j = 0; j < kExtBatchMax; ++j) sv[j] = j < a.nk ? SS[a.ssOff[j]] : 0.f;
+    for (int j = 0; j < kTimeBatchMax; ++j) sv[j] = j < a.nk ? SS[a.ssOff[j]] : 0.f;
     for (int e = a.eLo; e < a.eHi; ++e) {
         const long sh = 2L * a.lagDir * (e - a.hExt) * nzx;
         float m = IMG[nzx * e];
 #pragma unroll
-        for (int j = 0; j < kExtBatchMax; ++j)
+        for (int j = 0; j < kTimeBatchMax; ++j)
             if (j < a.nk && e >= a.lo[j] && e < a.hi[j]) m += sv[j] * W[a.wOff[j] - sh];
         IMG[nzx * e] = m;
     }
 }
 
-// The same two operations for a full interior batch: NK consecutive samples
-// (k_j = k0 + DIRK * j) with every lag |l| <= hExt <= HX usable.  The W
-// samples the batch touches, k0 - 2 hExt ... k0 + NK - 1 + 2 hExt, are read
-// once into a register window; slot r of the window holds W sample
-// kmin - 2 HX + r, so that every (sample, lag) pair has a compile-time
-// register index.  Each output receives the general kernels' operations in
-// their order (lags ascending; samples in batch order).
-template <int HX, int NK, int DIRK, int LAGDIR>
-__device__ __forceinline__ void time_window(const ExtBatchArgs& a, cgf* W, long nzx, float (&w)[NK + 4 * HX])
+// The same two operations for up to NK consecutive samples (k_j = k0 + DIRK *
+// j) and hExt <= HX.  The W samples the batch touches are read once into a
+// register window; slot r of the window holds W sample kmin - 2 HX + r, so
+// that every (sample, lag) pair has a compile-time register index.  Each
+// output receives the general kernels' operations in their order (lags
+// ascending; samples in batch order).  PART: fewer samples, or lags that reach
+// beyond the stored ones; every pair is then tested.  Lag direction -1 pairs
+// the slices the other way round.
+//
+// They are bound by memory: 16 samples and 10 lags read 56 slices of W and the
+// 21 of the image, which they also write.  32 samples read 72.  8 shots of 448 x
+// 976 points, 16 of them per launch: 384 us for 4 shots on each of two lanes, 4.2
+// TB/s; a partial batch took 1008 us on the general kernel.
+template <int HX, int NK, int DIRK, bool PART>
+__device__ __forceinline__ int time_window(const TimeBatchArgs& a, cgf* W, long nzx, float (&w)[NK + 4 * HX])
 {
-    const long kmin = DIRK > 0 ? a.wOff[0] / nzx : a.wOff[0] / nzx - (NK - 1);
-    const int h = a.hExt;
+    const int k0 = (int)(a.wOff[0] / nzx), kmin = DIRK > 0 ? k0 : k0 - (NK - 1), h = a.hExt;
 #pragma unroll
     for (int r = 0; r < NK + 4 * HX; ++r) {
-        const bool need = r >= 2 * (HX - h) && r < NK + 2 * HX + 2 * h;
-        w[r] = need ? W[(kmin - 2 * HX + r) * nzx] : 0.f;
+        const int k = kmin - 2 * HX + r;
+        const bool need = r >= 2 * (HX - h) && r < NK + 2 * HX + 2 * h && (!PART || (k >= 0 && k < a.nts));
+        w[r] = need ? W[k * nzx] : 0.f;
     }
+    return kmin;
 }
 
-template <int HX, int NK, int LAGDIR>
-__global__ void __launch_bounds__(64) k_time_ss_win(ExtBatchArgs a)
+template <int HX, int NK, bool PART>
+__global__ void __launch_bounds__(64) k_time_ss_win(TimeBatchArgs a)
 {
     const ShotSlot& S = a.slots[blockIdx.y];
     const long nz = a.nz, nzx = nz * a.nx;
@@ -2011,7 +2020,7 @@ __global__ void __launch_bounds__(64) k_time_ss_win(ExtBatchArgs a)
     if (iz >= a.nz - FAT) return;
     const long i = (long)ix * nz + iz;
     float w[NK + 4 * HX];
-    time_window<HX, NK, 1, LAGDIR>(a, G(S.W) + i, nzx, w);
+    const int kmin = time_window<HX, NK, 1, PART>(a, G(S.W) + i, nzx, w);
     const int h = a.hExt;
     cgf* M = G(a.mext) + i;
     float mv[2 * HX + 1];   // every lag's model value in flight before the arithmetic
@@ -2020,19 +2029,28 @@ __global__ void __launch_bounds__(64) k_time_ss_win(ExtBatchArgs a)
     float acc[NK];
 #pragma unroll
     for (int j = 0; j < NK; ++j) acc[j] = 0.f;
+    auto lags = [&](auto dir) {
+        constexpr int D = decltype(dir)::value;
 #pragma unroll
-    for (int l = -HX; l <= HX; ++l) {
-        if (l < -h || l > h) continue;
+        for (int l = -HX; l <= HX; ++l) {
+            if (l < -h || l > h) continue;
 #pragma unroll
-        for (int j = 0; j < NK; ++j) acc[j] += mv[l + HX] * w[j - 2 * LAGDIR * l + 2 * HX];
-    }
+            for (int j = 0; j < NK; ++j) {
+                const int k = kmin + j - 2 * D * l;
+                if (!PART || (j < a.nk && k >= 0 && k < a.nts)) acc[j] += mv[l + HX] * w[j - 2 * D * l + 2 * HX];
+            }
+        }
+    };
+    if (a.lagDir > 0) lags(std::integral_constant<int, 1>{});
+    else lags(std::integral_constant<int, -1>{});
     gf* SS = G(S.ss[0]) + i;
 #pragma unroll
-    for (int j = 0; j < NK; ++j) SS[a.ssOff[j]] = acc[j];
+    for (int j = 0; j < NK; ++j)
+        if (!PART || j < a.nk) SS[a.ssOff[j]] = acc[j];
 }
 
-template <int HX, int NK, int DIRK, int LAGDIR>
-__global__ void __launch_bounds__(64) k_time_img_win(ExtBatchArgs a)
+template <int HX, int NK, int DIRK, bool PART>
+__global__ void __launch_bounds__(64) k_time_img_win(TimeBatchArgs a)
 {
     const ShotSlot& S = a.slots[blockIdx.y];
     const long nz = a.nz, nzx = nz * a.nx;
@@ -2041,25 +2059,27 @@ __global__ void __launch_bounds__(64) k_time_img_win(ExtBatchArgs a)
     if (iz >= a.nz - FAT) return;
     const long i = (long)ix * nz + iz;
     float w[NK + 4 * HX];
-    time_window<HX, NK, DIRK, LAGDIR>(a, G(S.W) + i, nzx, w);
+    const int kmin = time_window<HX, NK, DIRK, PART>(a, G(S.W) + i, nzx, w);
     cgf* SS = G(S.ss[0]) + i;
-    gf* IMG = G(S.img) + i;
+    const int h = a.hExt;
+    gf* IMG = G(S.img) + i + nzx * h;
+    const long step = a.lagDir * nzx;                       // image slice of lag l: IMG + step * l
     float sv[NK];
 #pragma unroll
-    for (int j = 0; j < NK; ++j) sv[j] = SS[a.ssOff[j]];
-    const int h = a.hExt;
+    for (int j = 0; j < NK; ++j) sv[j] = !PART || j < a.nk ? SS[a.ssOff[j]] : 0.f;
     float m[2 * HX + 1];    // every lag's image value in flight before the arithmetic
 #pragma unroll
-    for (int l = -HX; l <= HX; ++l) m[l + HX] = (l >= -h && l <= h) ? IMG[nzx * (l + h)] : 0.f;
+    for (int l = -HX; l <= HX; ++l) m[l + HX] = (l >= -h && l <= h) ? IMG[step * l] : 0.f;
 #pragma unroll
     for (int l = -HX; l <= HX; ++l) {
         if (l < -h || l > h) continue;
 #pragma unroll
         for (int j = 0; j < NK; ++j) {
-            const int jj = DIRK > 0 ? j : NK - 1 - j;   // k_j - kmin
-            m[l + HX] += sv[j] * w[jj - 2 * LAGDIR * l + 2 * HX];
+            const int jj = DIRK > 0 ? j : NK - 1 - j;       // k_j - kmin
+            const int k = kmin + jj - 2 * l;
+            if (!PART || (j < a.nk && k >= 0 && k < a.nts)) m[l + HX] += sv[j] * w[jj - 2 * l + 2 * HX];
         }
-        IMG[nzx * (l + h)] = m[l + HX];
+        IMG[step * l] = m[l + HX];
     }
 }
 
@@ -2734,9 +2754,9 @@ hipError_t launch_img_acc_batch(const ImgAccArgs& a, int nshots, hipStream_t s)
 // The lag ranges must lie inside [0, 2 hExt] and reach W samples inside the
 // stored [0, nts) only (W is read at k - lagDir * 2 (e - hExt), extreme at
 // e = lo and e = hi - 1).
-static bool time_batch_ok(const ExtBatchArgs& a)
+static bool time_batch_ok(const TimeBatchArgs& a)
 {
-    if (a.nk < 1 || a.nk > kExtBatchMax || a.hExt < 0 || (a.lagDir != 1 && a.lagDir != -1)) return false;
+    if (a.nk < 1 || a.nk > kTimeBatchMax || a.hExt < 0 || (a.lagDir != 1 && a.lagDir != -1)) return false;
     if (a.eLo < 0 || a.eHi > 2 * a.hExt + 1 || a.eLo > a.eHi) return false;
     const long nzx = (long)a.nz * a.nx;
     for (int j = 0; j < a.nk; ++j) {
@@ -2752,51 +2772,74 @@ static bool time_batch_ok(const ExtBatchArgs& a)
     return true;
 }
 
-// A batch the register-window kernels take: kExtBatchMax samples k0 + dirK * j
-// with every lag usable (checked by time_batch_ok to stay inside [0, nts)).
-static bool time_batch_full(const ExtBatchArgs& a, int dirK)
+// Whether the register-window kernels take a batch: consecutive samples k0 +
+// dirK * j that use every lag whose W sample is stored (time_batch_ok has
+// checked that they use no other).
+static bool time_batch_window(const TimeBatchArgs& a, int dirK)
 {
-    if (a.nk != kExtBatchMax || a.hExt > 20 || a.eLo != 0 || a.eHi != 2 * a.hExt + 1) return false;
+    if (a.hExt > 20 || (a.hExt > 10 && a.nk > 16)) return false;
     const long nzx = (long)a.nz * a.nx;
-    for (int j = 0; j < a.nk; ++j)
-        if (a.lo[j] != 0 || a.hi[j] != 2 * a.hExt + 1 || a.wOff[j] != a.wOff[0] + dirK * j * nzx) return false;
+    for (int j = 0; j < a.nk; ++j) {
+        if (a.wOff[j] != a.wOff[0] + dirK * j * nzx) return false;
+        const long k = a.wOff[j] / nzx;
+        int lo = 0, hi = 2 * a.hExt + 1;
+        while (lo < hi && (k - 2L * a.lagDir * (lo - a.hExt) < 0 || k - 2L * a.lagDir * (lo - a.hExt) >= a.nts)) ++lo;
+        while (hi > lo && (k - 2L * a.lagDir * (hi - 1 - a.hExt) < 0 || k - 2L * a.lagDir * (hi - 1 - a.hExt) >= a.nts)) --hi;
+        if (lo < hi ? a.lo[j] != lo || a.hi[j] != hi : a.lo[j] < a.hi[j]) return false;
+    }
     return true;
 }
 
-template <int HX>
-static void time_ss_win(const ExtBatchArgs& a, dim3 g, hipStream_t s)
+// Of those, the batches of n samples whose every lag is stored.
+static bool time_batch_full(const TimeBatchArgs& a, int n)
 {
-    if (a.lagDir > 0) hipLaunchKernelGGL((k_time_ss_win<HX, kExtBatchMax, 1>), g, dim3(64), 0, s, a);
-    else hipLaunchKernelGGL((k_time_ss_win<HX, kExtBatchMax, -1>), g, dim3(64), 0, s, a);
+    if (a.nk != n) return false;
+    for (int j = 0; j < a.nk; ++j)
+        if (a.lo[j] != 0 || a.hi[j] != 2 * a.hExt + 1) return false;
+    return true;
 }
 
-template <int HX, int DIRK>
-static void time_img_win(const ExtBatchArgs& a, dim3 g, hipStream_t s)
+template <int HX, int NK>
+static void time_ss_win(const TimeBatchArgs& a, dim3 g, hipStream_t s)
 {
-    if (a.lagDir > 0) hipLaunchKernelGGL((k_time_img_win<HX, kExtBatchMax, DIRK, 1>), g, dim3(64), 0, s, a);
-    else hipLaunchKernelGGL((k_time_img_win<HX, kExtBatchMax, DIRK, -1>), g, dim3(64), 0, s, a);
+    if (time_batch_full(a, NK)) hipLaunchKernelGGL((k_time_ss_win<HX, NK, false>), g, dim3(64), 0, s, a);
+    else hipLaunchKernelGGL((k_time_ss_win<HX, NK, true>), g, dim3(64), 0, s, a);
 }
 
-hipError_t launch_time_ss_batch(const ExtBatchArgs& a, int nshots, hipStream_t s)
+template <int HX, int NK, int DIRK>
+static void time_img_win(const TimeBatchArgs& a, dim3 g, hipStream_t s)
+{
+    if (time_batch_full(a, NK)) hipLaunchKernelGGL((k_time_img_win<HX, NK, DIRK, false>), g, dim3(64), 0, s, a);
+    else hipLaunchKernelGGL((k_time_img_win<HX, NK, DIRK, true>), g, dim3(64), 0, s, a);
+}
+
+template <int HX, int NK>
+static void time_img_win(const TimeBatchArgs& a, int dirK, dim3 g, hipStream_t s)
+{
+    if (dirK > 0) time_img_win<HX, NK, 1>(a, g, s);
+    else time_img_win<HX, NK, -1>(a, g, s);
+}
+
+hipError_t launch_time_ss_batch(const TimeBatchArgs& a, int nshots, hipStream_t s)
 {
     if (!time_batch_ok(a)) return hipErrorInvalidValue;
     const dim3 g = column_grid(a.nz, a.nx, nshots);
-    if (!time_batch_full(a, 1)) hipLaunchKernelGGL(k_time_ss, g, dim3(64), 0, s, a);
-    else if (a.hExt <= 5) time_ss_win<5>(a, g, s);
-    else if (a.hExt <= 10) time_ss_win<10>(a, g, s);
-    else time_ss_win<20>(a, g, s);
+    if (!time_batch_window(a, 1)) hipLaunchKernelGGL(k_time_ss, g, dim3(64), 0, s, a);
+    else if (a.hExt <= 5) a.nk > 16 ? time_ss_win<5, 32>(a, g, s) : time_ss_win<5, 16>(a, g, s);
+    else if (a.hExt <= 10) a.nk > 16 ? time_ss_win<10, 32>(a, g, s) : time_ss_win<10, 16>(a, g, s);
+    else time_ss_win<20, 16>(a, g, s);
     return hipGetLastError();
 }
 
-hipError_t launch_time_img_batch(const ExtBatchArgs& a, int nshots, hipStream_t s)
+hipError_t launch_time_img_batch(const TimeBatchArgs& a, int nshots, hipStream_t s)
 {
     if (!time_batch_ok(a)) return hipErrorInvalidValue;
     const dim3 g = column_grid(a.nz, a.nx, nshots);
-    const int dirK = time_batch_full(a, 1) ? 1 : time_batch_full(a, -1) ? -1 : 0;
+    const int dirK = time_batch_window(a, 1) ? 1 : time_batch_window(a, -1) ? -1 : 0;
     if (dirK == 0) hipLaunchKernelGGL(k_time_img, g, dim3(64), 0, s, a);
-    else if (a.hExt <= 5) dirK > 0 ? time_img_win<5, 1>(a, g, s) : time_img_win<5, -1>(a, g, s);
-    else if (a.hExt <= 10) dirK > 0 ? time_img_win<10, 1>(a, g, s) : time_img_win<10, -1>(a, g, s);
-    else dirK > 0 ? time_img_win<20, 1>(a, g, s) : time_img_win<20, -1>(a, g, s);
+    else if (a.hExt <= 5) a.nk > 16 ? time_img_win<5, 32>(a, dirK, g, s) : time_img_win<5, 16>(a, dirK, g, s);
+    else if (a.hExt <= 10) a.nk > 16 ? time_img_win<10, 32>(a, dirK, g, s) : time_img_win<10, 16>(a, dirK, g, s);
+    else time_img_win<20, 16>(a, dirK, g, s);
     return hipGetLastError();
 }
 

@@ -92,21 +92,26 @@ struct StepArgs {
 // k_ext_img_tile): sample k's receiver / secondary-source slice is
 // ShotSlot::ss[0] + ssOff[k] and its source-wavefield slice W + wOff[k].
 constexpr int kExtBatchMax = 16;
-struct ExtBatchArgs {
+template <int N>
+struct ExtBatch {
     const ShotSlot* slots;
     const float* v2dt2;
     const float* mext;      // scaled extended model [nExt][nx][nz] (secondary sources)
     int nz, nx, hExt;
-    int nk;                 // samples in the batch, 1..kExtBatchMax
-    long ssOff[kExtBatchMax];
-    long wOff[kExtBatchMax];
+    int nk;                 // samples in the batch, 1..N
+    long ssOff[N];
+    long wOff[N];
     // time-lag extension: sample j uses lag slices [lo[j], hi[j]); eLo..eHi
     // spans them all; slice e reads W at k_j - lagDir * 2 (e - hExt)
-    int lo[kExtBatchMax], hi[kExtBatchMax];
+    int lo[N], hi[N];
     int eLo, eHi;
     int lagDir;             // +1 or -1
     int nts;                // coarse samples of W (bounds check of the time-lag batches)
 };
+using ExtBatchArgs = ExtBatch<kExtBatchMax>;
+// Time lags take twice as many, whose windows of W overlap by less.
+constexpr int kTimeBatchMax = 2 * kExtBatchMax;
+using TimeBatchArgs = ExtBatch<kTimeBatchMax>;
 
 // Image accumulation over a batch of coarse samples (k_img_acc_batch):
 // X.img += X.W[xOff[j]] * Y.W[yOff[j]] for j = 0 .. nk-1, in that order.
@@ -322,8 +327,8 @@ hipError_t launch_born_adj_finish(const ShotSlot* slots, int nshots, int ssR, co
 hipError_t launch_ext_ss_batch(const ExtBatchArgs& a, int nshots, hipStream_t s);
 // wemvaFwd: the WEMVA forward's imaging, (W_k[x-h] * ss_k[x+h]) * v2dt2[x+h]
 hipError_t launch_ext_img_batch(const ExtBatchArgs& a, int nshots, hipStream_t s, bool wemvaFwd = false);
-hipError_t launch_time_ss_batch(const ExtBatchArgs& a, int nshots, hipStream_t s);
-hipError_t launch_time_img_batch(const ExtBatchArgs& a, int nshots, hipStream_t s);
+hipError_t launch_time_ss_batch(const TimeBatchArgs& a, int nshots, hipStream_t s);
+hipError_t launch_time_img_batch(const TimeBatchArgs& a, int nshots, hipStream_t s);
 hipError_t launch_time_scale(const float* v2dt2, const float* refl, int sloth, float* out, int nz, int nx,
                              hipStream_t s);
 hipError_t launch_ext_adj_finish(const ShotSlot* slots, int nshots, const float* refl, int nz, int nx,

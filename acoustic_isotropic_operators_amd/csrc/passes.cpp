@@ -26,6 +26,23 @@ namespace aiso {
 
 namespace {
 
+// A batch of at most kExtBatchMax samples for the offset kernels.
+ExtBatchArgs offset_batch(const TimeBatchArgs& e)
+{
+    if (e.nk > kExtBatchMax) throw Error(AISO_ERR_STATE, "internal: too many samples in an offset batch");
+    ExtBatchArgs x{};
+    x.slots = e.slots;
+    x.v2dt2 = e.v2dt2;
+    x.mext = e.mext;
+    x.nz = e.nz; x.nx = e.nx; x.hExt = e.hExt;
+    x.nk = e.nk;
+    for (int j = 0; j < e.nk; ++j) {
+        x.ssOff[j] = e.ssOff[j];
+        x.wOff[j] = e.wOff[j];
+    }
+    return x;
+}
+
 class Call {
 public:
     Call(aiso_ctx* ctx, const Request& req) : c(ctx), q(req), p(ctx->p) {}
@@ -67,7 +84,7 @@ private:
     bool ring(unsigned mode, const StepArgs& sa);
     long ss_slot(int k) const { return (long)(k % ssSlices) * nzx; }
     long cap_off(int k) const { return (long)(k % capSlices) * nzx; }
-    void time_lags(ExtBatchArgs& e, int dir) const;
+    void time_lags(TimeBatchArgs& e, int dir) const;
     const aiso_device* rec_dev(int shot) const { return q.rec[q.nRec == 1 ? 0 : shot]; }
     DevGeom* rec_geom(int shot) const { return recG[q.nRec == 1 ? 0 : shot]; }
 
@@ -285,7 +302,10 @@ void Call::plan_batches()
     // The offset-extended passes keep a ring of coarse-rate slices per shot:
     // extK samples batched per imaging / secondary-source launch, plus the
     // one the time steps are writing or reading.
-    extK = std::min(c->extBatch, p.nts);
+    // Time lags of up to 10 take twice as many: 32 samples read 72 slices of
+    // W, 16 read 56 (adjoint of 8 shots of 333 x 871, 21 lags, 400 samples:
+    // 29.0 ms against 32.1).
+    extK = std::min(is_ext(q.op) && tlag && p.hExt <= 10 ? 2 * c->extBatch : c->extBatch, p.nts);
     ssSlices = is_ext(q.op) || tomo ? extK + 1 : 2;
     needImg = q.op == Op::BornAdj || q.op == Op::ExtAdj || q.op == Op::TomoAdj || wemva;
     // captured coarse samples kept per shot: the WEMVA forward's imaging and
@@ -457,7 +477,7 @@ void Call::init_step_args()
 // sample k - dir * 2 (e - hExt) lies in [0, nts)
 // (F/src/BornExtShotsGpuFunctions.cu:362-366, 374-378 for dir = +1;
 // F/src/tomoExtShotsGpuFunctions.cu:2630-2633 for dir = -1).
-void Call::time_lags(ExtBatchArgs& e, int dir) const
+void Call::time_lags(TimeBatchArgs& e, int dir) const
 {
     e.nts = p.nts;
     e.lagDir = dir;
@@ -983,7 +1003,7 @@ void Call::passes_tomo()
     };
     enum { SS_EXT, SS_MUL, SS_ADJ };   // ring producers
     auto produce = [&](int kind, const ShotSlot* from, const float* scale, int k0, int n) {
-        ExtBatchArgs e{};
+        TimeBatchArgs e{};
         e.slots = from;
         e.v2dt2 = base.v2dt2;
         e.mext = scale;
@@ -995,12 +1015,12 @@ void Call::passes_tomo()
         }
         if (kind != SS_MUL && tlag) time_lags(e, kind == SS_EXT ? 1 : -1);
         lanes([&](int s0, int cnt, hipStream_t st) {
-            ExtBatchArgs el = e;
+            TimeBatchArgs el = e;
             el.slots = from + s0;
-            if (kind == SS_MUL) HIPC(launch_mul_batch(el, cnt, st));
+            if (kind == SS_MUL) HIPC(launch_mul_batch(offset_batch(el), cnt, st));
             else if (tlag) HIPC(launch_time_ss_batch(el, cnt, st));   // imagingTimeFwdGpu / imagingTimeTomoAdjGpu
-            else if (kind == SS_EXT) HIPC(launch_ext_ss_batch(el, cnt, st));
-            else HIPC(launch_tomo_adj_ss(el, cnt, st));
+            else if (kind == SS_EXT) HIPC(launch_ext_ss_batch(offset_batch(el), cnt, st));
+            else HIPC(launch_tomo_adj_ss(offset_batch(el), cnt, st));
         });
     };
     // Forward in time.  ssKind >= 0: inject ring samples made from `from`'s
@@ -1228,7 +1248,7 @@ void Call::passes_tomo()
         std::vector<int> pend;
         auto flush = [&](bool wemvaFwd) {
             if (pend.empty()) return;
-            ExtBatchArgs e{};
+            TimeBatchArgs e{};
             e.slots = wemvaFwd ? dSlotsJ : dSlotsI;
             e.v2dt2 = base.v2dt2;
             e.nz = p.nz; e.nx = p.nx; e.hExt = p.hExt;
@@ -1242,10 +1262,10 @@ void Call::passes_tomo()
             if (tlag) time_lags(e, wemvaFwd ? -1 : 1);   // imagingWemvaTimeAdjGpu / imagingTimeAdjGpu
             const ShotSlot* base0 = e.slots;
             lanes([&](int s0, int cnt, hipStream_t st) {
-                ExtBatchArgs el = e;
+                TimeBatchArgs el = e;
                 el.slots = base0 + s0;
                 if (tlag) HIPC(launch_time_img_batch(el, cnt, st));
-                else HIPC(launch_ext_img_batch(el, cnt, st, wemvaFwd));
+                else HIPC(launch_ext_img_batch(offset_batch(el), cnt, st, wemvaFwd));
             });
             pend.clear();
         };
@@ -1325,7 +1345,7 @@ void Call::pass_forward()
     int nextSS = 0;
     auto ext_ss_upto = [&](int upto) {
         while (nextSS <= upto) {
-            ExtBatchArgs e{};
+            TimeBatchArgs e{};
             e.slots = dSlots;
             e.v2dt2 = base.v2dt2;
             e.mext = mtil;
@@ -1340,10 +1360,10 @@ void Call::pass_forward()
                 int k0, cnt;
                 lane_range(nb, c->curLanes, l, k0, cnt);
                 if (cnt == 0) continue;
-                ExtBatchArgs el = e;
+                TimeBatchArgs el = e;
                 el.slots = dSlots + k0;
                 if (tlag) HIPC(launch_time_ss_batch(el, cnt, lane_stream(c, l)));
-                else HIPC(launch_ext_ss_batch(el, cnt, lane_stream(c, l)));
+                else HIPC(launch_ext_ss_batch(offset_batch(el), cnt, lane_stream(c, l)));
             }
             nextSS += e.nk;
         }
@@ -1426,7 +1446,7 @@ void Call::pass_adjoint()
         int lanesNow = c->curLanes;
         auto ext_img_flush = [&] {
             if (pend.empty()) return;
-            ExtBatchArgs e{};
+            TimeBatchArgs e{};
             e.slots = sl;
             e.v2dt2 = base.v2dt2;
             e.nz = p.nz; e.nx = p.nx; e.hExt = p.hExt;
@@ -1442,11 +1462,11 @@ void Call::pass_adjoint()
                 int k0, cnt;
                 lane_range(nbr, lanesNow, l, k0, cnt);
                 if (cnt == 0) continue;
-                ExtBatchArgs el = e;
+                TimeBatchArgs el = e;
                 el.slots = sl + k0;
                 hipStream_t ls = lanesNow > 1 ? lane_stream(c, l) : s;
                 if (tlag) HIPC(launch_time_img_batch(el, cnt, ls));
-                else HIPC(launch_ext_img_batch(el, cnt, ls));
+                else HIPC(launch_ext_img_batch(offset_batch(el), cnt, ls));
             }
             pend.clear();
         };
