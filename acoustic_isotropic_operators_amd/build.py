@@ -1,6 +1,6 @@
 """Build the native parts of the package in-tree.
 
-* ``libaiso.so``: the HIP engine (kernels.hip, wide.hip, steps.hip, engine.cpp, host.cpp) for gfx950,
+* ``libaiso.so``: the HIP engine (kernels.hip, wide.hip, steps.hip, ext.hip, engine.cpp, host.cpp) for gfx950,
   exporting the C-ABI declared in ``include/aiso.h``;
 * the pybind11 modules ``pyAcoustic_iso_float_{nl,born,born_ext,tomo,wemva}`` that mirror the
   reference's module names on top of that C-ABI.
@@ -47,7 +47,7 @@ def build_lib():
     bdir = os.path.join(PKG, "_build")
     os.makedirs(bdir, exist_ok=True)
     cmds, objs = [], []
-    for src in ("kernels.hip", "wide.hip", "steps.hip", "noalloc.hip", "engine.cpp", "passes.cpp", "windows.cpp", "host.cpp"):
+    for src in ("kernels.hip", "wide.hip", "steps.hip", "ext.hip", "noalloc.hip", "engine.cpp", "passes.cpp", "windows.cpp", "host.cpp"):
         obj = os.path.join(bdir, src.replace(".", "_") + ".o")
         lang = [] if src.endswith(".hip") else ["-x", "hip"]
         # the kernels' register, scratch and occupancy figures, kept for the tests

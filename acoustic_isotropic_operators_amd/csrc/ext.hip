@@ -1,0 +1,138 @@
+// ext.hip -- secondary sources of the offset extension with four z-points per
+// lane.
+//
+// What bounds them: the latency of one sample's pieces per barrier, with two
+// workgroups of 8 waves per CU (230 vector instructions per 256 points and
+// sample, 168 of them the products and sums; no LDS conflicts).  All offsets
+// are computed without a test, those beyond 2 hExt on zeros: with a branch per
+// offset every LDS read was waited for.  64 x 32 tiles stage 2.25 times their
+// points, the one-point kernels' 64 x 16 ones 3.5 times.
+// Extended forward, 6 shots of 500 x 1200, 21 offsets, 300 samples: 27.2 ms,
+// one point per lane 30.3; tomographic adjoint, 6 shots of 300 x 700: 33.1 ms,
+// 37.1.  Up to 11 offsets both take the same time, and the one-point kernels
+// stay.
+#include <hip/hip_runtime.h>
+
+#include "wide.hpp"
+
+namespace aiso {
+
+namespace {
+
+constexpr int kTZ = 64, kTX = 32, kQ = kTZ / 4, kThreads = kQ * kTX;
+constexpr int kShots = 2;   // shots per workgroup, which share its model values
+
+// For the nk samples of each shot, into ss[0] + ssOff[k], over the offsets h =
+// -hExt .. hExt in order:
+//   ss_k[x] = v2dt2[x] * sum m[h][x-h] * W_k[x-2h]              (k_ext_ss_tile)
+//   TOMO: ss_k[x] = sum (m[h][x+h] * W_k[x+2h]) * v2dt2[x+2h]    (k_tomo_adj_ss_tile)
+// Each thread owns four rows of one column and keeps its model values in
+// registers; W passes through LDS in 16-byte pieces, the next sample's loaded
+// while the current one is computed, into the other half: one barrier per
+// sample.  Offsets that leave the interior have a model value of zero.
+template <int HX, bool TOMO>
+__global__ __launch_bounds__(kThreads) void k_offset_ss(ExtBatchArgs a, int nshots, int nbx, int nbz, int nby)
+{
+    constexpr int NE = 2 * HX + 1, LW = kTX + 4 * HX, SZ = LW * kTZ, KU = (LW * kQ + kThreads - 1) / kThreads;
+    __shared__ __attribute__((aligned(16))) float lds[(TOMO ? 3 : 2) * SZ];
+    const int l = xcd_logical(blockIdx.x, gridDim.x);
+    if (l >= nbx * nbz * nby) return;                                           // padding blocks (block-uniform)
+    const int bx = l % nbx, bz = l / nbx % nbz, by = l / nbx / nbz, t = threadIdx.x;
+    const int hExt = a.hExt, ne = 2 * hExt + 1, lw = kTX + 4 * hExt, nzi = a.nz - 2 * FAT;
+    const int z0 = bz * kTZ, x0 = FAT + bx * kTX;                               // interior row, grid column
+    const long nzx = (long)a.nz * a.nx;
+    // Offset e takes LDS column c + 2e (TOMO) or c + 4 HX - 2e, whatever hExt
+    // is: column j is grid column x0 - 2 hExt + j (TOMO) or x0 + 2 hExt - 4 HX
+    // + j.  Columns outside the interior and those that only offsets beyond
+    // 2 hExt take are zero.
+    unsigned off[KU];
+    bool in[KU];
+    f4 pre[KU];
+#pragma unroll
+    for (int k = 0; k < KU; ++k) {
+        const int u = t + k * kThreads, j = u / kQ - (TOMO ? 0 : 4 * (HX - hExt)), q = u % kQ, gx = x0 - 2 * hExt + j;
+        in[k] = j >= 0 && j < lw && gx >= FAT && gx < a.nx - FAT && z0 + 4 * q < nzi;
+        off[k] = in[k] ? 4u * (unsigned)(gx * a.nz + FAT + z0 + 4 * q) : 0u;
+        pre[k] = (f4)0.f;
+    }
+    auto fetch = [&](cgf* w) {
+#pragma unroll
+        for (int k = 0; k < KU; ++k)
+            if (in[k]) pre[k] = ld4(w, off[k]);
+    };
+    auto store = [&](float* to) {
+#pragma unroll
+        for (int k = 0; k < KU; ++k)
+            if (t + k * kThreads < LW * kQ) *(f4a*)&to[4 * (t + k * kThreads)] = pre[k];
+    };
+    const int sh0 = by * kShots, nsh = imin(kShots, nshots - sh0);
+    if constexpr (TOMO) {
+        fetch(G(a.v2dt2));
+        store(lds + 2 * SZ);
+    }
+    static_assert(kShots == 2, "the bases of two shots, read before the first store");
+    cgf* W0 = G(a.slots[sh0].W);
+    cgf* W1 = G(a.slots[sh0 + nsh - 1].W);
+    gf* S0 = G(a.slots[sh0].ss[0]);
+    gf* S1 = G(a.slots[sh0 + nsh - 1].ss[0]);
+    fetch(W0 + a.wOff[0]);
+
+    const int zq = t % kQ, c = t / kQ, x = x0 + c;
+    const bool ok = z0 + 4 * zq < nzi && x < a.nx - FAT;
+    const unsigned o = 4u * (unsigned)(x * a.nz + FAT + z0 + 4 * zq);
+    const int lo = TOMO ? max(-hExt, FAT + hExt - x) : max(-hExt, x + 1 + FAT + hExt - a.nx);
+    const int hi = TOMO ? imin(a.nx - 1 - FAT - x - hExt, hExt) : imin(x - hExt - FAT, hExt);
+    f4 mv[NE], vs = (f4)0.f;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+        const int h = e - hExt;
+        mv[e] = (f4)0.f;
+        if (ok && e < ne && h >= lo && h <= hi)
+            mv[e] = ld4(G(a.mext) + nzx * e + (long)(TOMO ? h : -h) * a.nz, o);
+    }
+    if (!TOMO && ok) vs = ld4(G(a.v2dt2), o);
+    store(lds);
+    __syncthreads();
+    const int j0 = (TOMO ? c : c + 4 * HX) * kTZ + 4 * zq;
+    int b = 0;
+    for (int q = 0; q < nsh; ++q) {
+        cgf* W = q ? W1 : W0;
+        gf* ss = q ? S1 : S0;
+        for (int k = 0; k < a.nk; ++k) {
+            const bool more = k + 1 < a.nk || q + 1 < nsh;
+            if (more) fetch(k + 1 < a.nk ? W + a.wOff[k + 1] : W1 + a.wOff[0]);
+            const float* w = &lds[b * SZ + j0];
+            const float* v = &lds[2 * SZ + j0];
+            f4 acc = (f4)0.f;
+#pragma unroll
+            for (int e = 0; e < NE; ++e) {
+                if constexpr (TOMO) acc += (mv[e] * *(const f4a*)(w + 2 * e * kTZ)) * *(const f4a*)(v + 2 * e * kTZ);
+                else acc += mv[e] * *(const f4a*)(w - 2 * e * kTZ);
+            }
+            if (ok) st4(ss + a.ssOff[k], o, TOMO ? acc : acc * vs);
+            if (more) store(lds + (b ^ 1) * SZ);
+            __syncthreads();
+            b ^= 1;
+        }
+    }
+}
+
+template <bool TOMO>
+hipError_t launch(const ExtBatchArgs& a, int nshots, hipStream_t s)
+{
+    const int nzi = a.nz - 2 * FAT, nxi = a.nx - 2 * FAT;
+    if (a.nk < 1 || a.nk > kExtBatchMax || a.hExt < 0 || a.hExt > kOffsetSsMax || !wide_grid_ok(a.nz, a.nx))
+        return hipErrorInvalidValue;
+    if (nzi <= 0 || nxi <= 0 || nshots < 1) return hipSuccess;
+    const int bx = (nxi + kTX - 1) / kTX, bz = (nzi + kTZ - 1) / kTZ, by = (nshots + kShots - 1) / kShots;
+    const dim3 g((bx * bz * by + 7) / 8 * 8), n(kThreads);
+    hipLaunchKernelGGL((k_offset_ss<kOffsetSsMax, TOMO>), g, n, 0, s, a, nshots, bx, bz, by);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_offset_ss(const ExtBatchArgs& a, int nshots, hipStream_t s) { return launch<false>(a, nshots, s); }
+hipError_t launch_offset_ss_tomo(const ExtBatchArgs& a, int nshots, hipStream_t s) { return launch<true>(a, nshots, s); }
+
+}  // namespace aiso

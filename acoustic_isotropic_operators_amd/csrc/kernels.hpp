@@ -327,6 +327,12 @@ hipError_t launch_born_adj_finish(const ShotSlot* slots, int nshots, int ssR, co
 hipError_t launch_ext_ss_batch(const ExtBatchArgs& a, int nshots, hipStream_t s);
 // wemvaFwd: the WEMVA forward's imaging, (W_k[x-h] * ss_k[x+h]) * v2dt2[x+h]
 hipError_t launch_ext_img_batch(const ExtBatchArgs& a, int nshots, hipStream_t s, bool wemvaFwd = false);
+// launch_ext_ss_batch and launch_tomo_adj_ss with four z-points per lane
+// (ext.hip), hExt up to kOffsetSsMax, for grids wide_grid_ok accepts; used
+// beyond kOffsetSsMin.
+constexpr int kOffsetSsMin = 5, kOffsetSsMax = 10;
+hipError_t launch_offset_ss(const ExtBatchArgs& a, int nshots, hipStream_t s);
+hipError_t launch_offset_ss_tomo(const ExtBatchArgs& a, int nshots, hipStream_t s);
 hipError_t launch_time_ss_batch(const TimeBatchArgs& a, int nshots, hipStream_t s);
 hipError_t launch_time_img_batch(const TimeBatchArgs& a, int nshots, hipStream_t s);
 hipError_t launch_time_scale(const float* v2dt2, const float* refl, int sloth, float* out, int nz, int nx,
