@@ -109,7 +109,7 @@ struct ExtBatch {
     int nts;                // coarse samples of W (bounds check of the time-lag batches)
 };
 using ExtBatchArgs = ExtBatch<kExtBatchMax>;
-// Time lags take twice as many, whose windows of W overlap by less.
+// Time lags and the imaging of ext.hip take twice as many.
 constexpr int kTimeBatchMax = 2 * kExtBatchMax;
 using TimeBatchArgs = ExtBatch<kTimeBatchMax>;
 
@@ -332,6 +332,7 @@ hipError_t launch_ext_img_batch(const ExtBatchArgs& a, int nshots, hipStream_t s
 // beyond kOffsetSsMin.
 constexpr int kOffsetSsMin = 5, kOffsetSsMax = 10;
 hipError_t launch_offset_ss(const ExtBatchArgs& a, int nshots, hipStream_t s);
+hipError_t launch_offset_img(const TimeBatchArgs& a, int nshots, hipStream_t s);   // launch_ext_img_batch, not wemvaFwd
 hipError_t launch_offset_ss_tomo(const ExtBatchArgs& a, int nshots, hipStream_t s);
 hipError_t launch_time_ss_batch(const TimeBatchArgs& a, int nshots, hipStream_t s);
 hipError_t launch_time_img_batch(const TimeBatchArgs& a, int nshots, hipStream_t s);

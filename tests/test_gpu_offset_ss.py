@@ -1,8 +1,9 @@
-"""The secondary sources of the offset extension with four z-points per lane
-(more than 11 offsets) give the float oracle's results bit for bit: interior
-sizes that leave remainders of the 64 x 32 tiles, grids narrower than the
-offsets' reach, offsets up to the kernels' bound and beyond, odd shot counts
-(a workgroup takes two) and batches of samples that do not divide the record."""
+"""The secondary sources and the imaging of the offset extension with four
+z-points per lane (more than 11 offsets) give the float oracle's results bit
+for bit: interior sizes that leave remainders of the 64 x 32 and 64 x 28 tiles,
+grids narrower than the offsets' reach, offsets up to the kernels' bound and
+beyond, odd shot counts (a workgroup takes two) and batches of samples, odd and
+even, that do not divide the record."""
 import numpy as np
 import pytest
 
@@ -36,6 +37,10 @@ def test_extended_and_tomographic(nzi, nxi, shots, nExt, batch):
     assert np.abs(ref).max() > 0
     np.testing.assert_array_equal(d, ref)
     ctx.set_ext_reflectivity(m)
+    ext = np.zeros_like(m)
+    da = rng.standard_normal(d.shape).astype(np.float32)
+    ctx.bornext_adjoint(ext, da, srcs, wav, recs)
+    np.testing.assert_array_equal(ext, O.bornext_adjoint(c.grid, c.vel, os_, [wav], or_, da, "f"))
     dr = rng.standard_normal(d.shape).astype(np.float32)
     img = np.zeros((c.nx, c.nz), np.float32)
     ctx.tomo_adjoint(img, dr, srcs, wav, recs)
