@@ -69,8 +69,7 @@ struct aiso_batch {
     int nSrcDev = 0;
     // the configuration the device tables hold, and the graphs captured with it
     aiso::BatchConfig cfg, prepared;
-    bool cfgSet = false;              // cfg was set or tuned; else the tile width of the tables is chosen here
-    int tx = 0;                       // tile width of the device tables
+    bool cfgSet = false;              // cfg was set or tuned; else run_config chooses
     bool isPrepared = false;
     std::vector<int> groupTiles;      // tiles of each launch group
     std::vector<long> groupPts;       // interior points of each launch group
@@ -127,24 +126,31 @@ int n_groups(const aiso_batch* b, const BatchConfig& c)
     return (n + spl - 1) / spl;
 }
 
-// Tile width of a batch whose configuration the caller left open.  A 32 x 32
-// tile reads 1.6 times its points to stage the halo, a 32 x 16 tile 2.1 times,
-// but makes twice the workgroups, which few points need.  Time of 300 samples
-// on 32 x 32 / 32 x 16 tiles (MI355X): 24 windows of 400 x 300-1500 points 19.7 /
-// 22.6 ms, 40 of 287 x 900 17.4 / 20.3 ms; 3 of 400 x 1500 (1600 tiles of 32 x 32)
-// 4.61 / 4.54 ms, 6 of 150 x 700 (830) 3.61 / 3.42 ms.
-int open_tile_width(const aiso_batch* b)
+// The configuration a call runs: the caller's, or where the caller left it
+// open, from 4096 tiles of 32 x 32 on, those tiles and two launch groups, whose
+// lanes fill each other's launch tails.  A 32 x 32 tile reads 1.6 times its
+// points to stage the halo, a 32 x 16 tile 2.1 times, but makes twice the
+// workgroups, which few points need.  Time of 300 samples (MI355X), 32 x 32 tiles
+// in two groups / in one / 32 x 16 tiles: 24 windows of 400 x 300-1500 points
+// 18.8 / 19.8 / 22.6 ms, 40 of 287 x 900 16.7 / 17.6 / 20.3 ms; 3 of 400 x 1500
+// (1600 tiles of 32 x 32) - / 4.61 / 4.54 ms, 6 of 150 x 700 (830) - / 3.61 / 3.42.
+BatchConfig run_config(const aiso_batch* b)
 {
+    BatchConfig c = b->cfg;
+    if (b->cfgSet) return c;
     long tiles = 0;
     for (auto& W : b->win) tiles += window_tiles(W->p, 32, 32);
-    return tiles >= 4096 ? 32 : 16;
+    if (tiles >= 4096) {
+        c.tx = 32;
+        c.spl = ((int)b->win.size() + 1) / 2;
+    }
+    return c;
 }
 
 // Device tables of configuration c: slots, window descriptors, tile map.
-void prepare(aiso_batch* b, const BatchConfig& c, bool set)
+void prepare(aiso_batch* b, const BatchConfig& c)
 {
-    const int tx = set ? c.tx : open_tile_width(b);
-    if (b->isPrepared && b->prepared == c && b->tx == tx) return;
+    if (b->isPrepared && b->prepared == c) return;
     if (c.tz != 32 && c.tz != 64) throw Error(AISO_ERR_PARAM, "tile tz must be 32 or 64");
     if (c.tx != 16 && c.tx != 32) throw Error(AISO_ERR_PARAM, "tile tx must be 16 or 32");
     if (c.spl < 0 || c.persist < 0) throw Error(AISO_ERR_PARAM, "windows per launch and workgroups per CU are >= 0");
@@ -161,8 +167,8 @@ void prepare(aiso_batch* b, const BatchConfig& c, bool set)
         long pts = 0;
         for (int w = g0; w < std::min(n, g0 + spl); ++w) {
             aiso_batch::Win& W = *b->win[w];
-            WinGeom* sg = win_geom(b, W, W.src, true, c.tz, tx);
-            WinGeom* rg = win_geom(b, W, W.rec, false, c.tz, tx);
+            WinGeom* sg = win_geom(b, W, W.src, true, c.tz, c.tx);
+            WinGeom* rg = win_geom(b, W, W.rec, false, c.tz, c.tx);
             ShotSlot& S = slots[w];
             std::memset(&S, 0, sizeof(S));
             S.p[0] = b->pairs.as<float>() + b->pairOff[w];
@@ -178,7 +184,7 @@ void prepare(aiso_batch* b, const BatchConfig& c, bool set)
             D.nz = W.p.nz;
             D.nx = W.p.nx;
             D.tilesZ = (W.p.nz - 2 * kFat + c.tz - 1) / c.tz;
-            D.ntiles = (int)window_tiles(W.p, c.tz, tx);
+            D.ntiles = (int)window_tiles(W.p, c.tz, c.tx);
             for (int t = 0; t < D.ntiles; ++t) map.push_back(make_int2(w - g0, t));
             tiles += D.ntiles;
             pts += W.interior();
@@ -191,7 +197,6 @@ void prepare(aiso_batch* b, const BatchConfig& c, bool set)
     upload(b->tileMap, map, b->stream);
     HIPC(hipStreamSynchronize(b->stream));   // the host vectors go out of scope
     b->prepared = c;
-    b->tx = tx;
     b->isPrepared = true;
     b->graphs.assign(b->groupTiles.size(), nullptr);
 }
@@ -286,7 +291,7 @@ void launch_steps(aiso_batch* b, int g, int t0, int t1, hipStream_t st, hipEvent
         w.a.ff = f[h + it2];
         hipEvent_t a0 = t == t0 ? e0 : nullptr, a1 = t == t1 - 1 ? e1 : nullptr;
         if (a0 && !a1) HIPC(hipEventRecord(a0, st));
-        HIPC(launch_step_windows(MODE_NL_FWD, b->prepared.tz, b->tx, grid, w, st,
+        HIPC(launch_step_windows(MODE_NL_FWD, b->prepared.tz, b->prepared.tx, grid, w, st,
                                  a0 && a1 ? a0 : nullptr, a0 && a1 ? a1 : nullptr));
         if (a1 && !a0) HIPC(hipEventRecord(a1, st));
     }
@@ -367,7 +372,7 @@ void batch_nl_forward(aiso_batch* b, int add, const float* const* model, int nMo
         HIPC(hipEventRecord(b->evIn, nullptr));
         HIPC(hipStreamWaitEvent(s, b->evIn, 0));
     }
-    prepare(b, b->cfg, b->cfgSet);
+    prepare(b, run_config(b));
     const FdParams& p0 = b->win[0]->p;
     const size_t modelN = (size_t)b->nSrcDev * p0.nts;
     // source traces of every window, staged through pinned memory
@@ -428,7 +433,7 @@ void batch_nl_forward(aiso_batch* b, int add, const float* const* model, int nMo
 // point-update.
 double time_config(aiso_batch* b, const BatchConfig& c, int steps)
 {
-    prepare(b, c, true);
+    prepare(b, c);
     const int G = (int)b->groupTiles.size();
     const int L = lanes_for(b, c, G);
     hipStream_t s = b->stream;
@@ -660,7 +665,7 @@ aiso_status aiso_batch_info(const aiso_batch* b, int* nWin, int* launchGroups, l
     long long pts = 0;
     for (auto& W : b->win) pts += (long long)W->interior() * (W->p.ntw - 1);
     if (nWin) *nWin = (int)b->win.size();
-    if (launchGroups) *launchGroups = b->win.empty() ? 0 : n_groups(b, b->cfg);
+    if (launchGroups) *launchGroups = b->win.empty() ? 0 : n_groups(b, run_config(b));
     if (pointUpdates) *pointUpdates = pts;
     if (lastMs) *lastMs = b->lastMs;
     if (captureMs) *captureMs = b->lastCaptureMs;
