@@ -302,6 +302,16 @@ StepArgs lane_args(const StepArgs& a, int k0, int cnt)
     return y;
 }
 
+// Lanes for a batch, unless the caller chose: one where a step of all its shots
+// is so short that submitting two launches (3.6 us each) takes longer.  Time with one lane / with
+// two (MI355X), by the points of a step: 0.3 to 0.8 million 0.72-0.93, 0.93 to 1.3
+// million 0.94-0.98, 1.6 to 1.9 million 1.04-1.13.
+int lanes_for(const aiso_ctx* c, int nShot, int fields)
+{
+    if (!c->lanesSet && (double)c->p.interior() * nShot * fields < 1.3e6) return 1;
+    return std::max(1, std::min(c->lanes, nShot));
+}
+
 hipStream_t lane_stream(const aiso_ctx* c, int l) { return c->curLanes > 1 ? c->lane[l] : c->stream; }
 
 void ensure_lanes(aiso_ctx* c)
@@ -732,7 +742,7 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
             launch_timed(c, mode, AISO_K_SRC, x);
             if (maxSrcRing > 0) ring_lanes(M_INJ_SIG, x, maxSrcRing);
         };
-        c->curLanes = std::max(1, std::min(c->lanes, nb));
+        c->curLanes = steps >= 0 ? std::max(1, std::min(c->lanes, nb)) : lanes_for(c, nb, 1);
         if (c->curLanes > 1) ensure_lanes(c);
         fork_lanes(c);
         // One fine step t from slice cur, or several in one launch: x.n steps
@@ -996,6 +1006,7 @@ aiso_status aiso_ctx_set_option(aiso_ctx* c, const char* key, int value)
         else if (k == "lanes") {
             if (value < 1 || value > 4) throw Error(AISO_ERR_PARAM, "lanes must be 1..4");
             c->lanes = value;
+            c->lanesSet = true;
         }
         else if (k == "tileFwd" || k == "tileAdj") {   // tz * 100 + tx
             const int tz = value / 100, tx = value % 100;

@@ -149,6 +149,7 @@ struct aiso_ctx {
     // MI355X two lanes raise the Born benchmark from 279 to 296 Gpts/s;
     // three and four lanes measured slower than one.
     int lanes = 2;
+    bool lanesSet = false;              // the caller chose them
     int extBatch = 16;                  // coarse samples per offset-imaging / secondary-source launch
     int curLanes = 1;                   // lanes of the call in progress
     std::vector<hipStream_t> lane;
@@ -247,6 +248,7 @@ hipEvent_t pooled_event(aiso_ctx* c);
 void wait_default_stream(aiso_ctx* c);
 void lane_range(int nshots, int lanes, int l, int& k0, int& cnt);
 StepArgs lane_args(const StepArgs& a, int k0, int cnt);
+int lanes_for(const aiso_ctx* c, int nShot, int fields);
 hipStream_t lane_stream(const aiso_ctx* c, int l);
 void ensure_lanes(aiso_ctx* c);
 void fork_lanes(aiso_ctx* c);

@@ -571,7 +571,7 @@ void Call::begin_batch(int first, int count)
     a = base;
     a.nshots = nb;
     a.gridLogical = a.ntiles * nb;
-    c->curLanes = pair2 || adj2 ? 1 : std::max(1, std::min(c->lanes, nb));
+    c->curLanes = pair2 || adj2 ? 1 : lanes_for(c, nb, lockstep ? 2 : 1);
     if (c->curLanes > 1) ensure_lanes(c);
 }
 
@@ -1296,9 +1296,11 @@ int Call::run_steps(int config, unsigned mode, int kind, StepsArgs x)
 {
     const int T = p.ntw - 1;
     const bool adj = mode & M_ADJ;
-    // One stream where the workgroups of all shots fit two rounds: the lanes'
+    // One stream where the workgroups of all shots run at once: the lanes'
     // launches would only cost the host.
-    const int lanes = (long)x.ntiles * nb > 512 ? c->curLanes : 1;
+    const int before = c->curLanes, lanes = (long)x.ntiles * nb > 256 ? std::max(1, std::min(c->lanes, nb)) : 1;
+    c->curLanes = lanes;
+    if (lanes > 1) ensure_lanes(c);
     hipEvent_t passT = lanes > 1 ? pass_timer_begin(c) : nullptr;
     if (lanes > 1) fork_lanes(c);
     for (int done = 0; done < T; done += x.n) {
@@ -1323,6 +1325,7 @@ int Call::run_steps(int config, unsigned mode, int kind, StepsArgs x)
     }
     if (lanes > 1) join_lanes(c);
     pass_timer_end(c, passT, kind, double(p.interior()) * nb * T, T);
+    c->curLanes = before;
     return x.pair;
 }
 
