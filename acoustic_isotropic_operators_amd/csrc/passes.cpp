@@ -360,16 +360,19 @@ void Call::plan_batches()
     B = std::min(B, q.nShot);
     B = (q.nShot + (q.nShot + B - 1) / B - 1) / ((q.nShot + B - 1) / B);   // same batch count, balanced sizes
     c->batchUsed = B;
-    // The lines for the largest tile, by its workgroups: microseconds per step,
-    // or time of the call, with it and in one-step launches.
-    //   nonlinear     320: 6.3 / 7.8   400: 7.3 / 7.8
-    //   its adjoint   240: 4.1 / 7.0   504: 8.4 / 7.4
-    //   Born, sub 3, 4: 240: 0.73 of the time, 400: 0.97, 504: 0.86
-    //   its adjoint's receiver pass, which moves the image once per launch:
-    //     640: 0.82, 840: 0.90, 1680: 0.95, 2952: 0.98, 4200: 1.03
+    // The lines for the largest tile, by its workgroups, with the time of the
+    // call in one-step launches as 1:
+    //   nonlinear                     400: 0.70   504: 0.76   840: 0.95   1176: 1.02   1680: 1.12
+    //   its adjoint                   400: 0.70   504: 0.98   840: 0.97   1176: 1.05   1680: 1.20
+    //   Born with captures per step   504: 0.73   840: 0.78  1260: 0.83   3360: 0.94   3690: 0.93
+    //   its adjoint's source pass     504: 0.85  1680: 0.89  3360: 0.96
+    //   Born adjoint, window, both    504: 0.79  1008: 0.84  1344: 0.88   1680: 0.93   2520: 1.03
+    //   its receiver pass alone, whose image moves once per launch
+    //                                 640: 0.82   840: 0.90  1680: 0.95   2952: 0.98   4200: 1.03
     if (multi && !lockstep) {
-        if (is_born(q.op)) stepsSrc = steps_config(B, 512);
-        if (q.op != Op::BornAdj) steps = steps_config(B, q.op == Op::NlAdj ? 256 : 512);
+        const long any = 1L << 40;
+        if (is_born(q.op)) stepsSrc = steps_config(B, win ? 1700 : any);
+        if (q.op != Op::BornAdj) steps = steps_config(B, q.op == Op::BornFwd && !win ? any : 1000);
         else if (win && c->batchRec == 0) steps = steps_config(B, 3000);
     }
     if (pairSlices == 4 && !pair2 && !adj2 && steps < 0 && stepsSrc < 0) {
