@@ -290,8 +290,8 @@ void Call::plan_batches()
     adj2 = q.op == Op::BornAdj && p.sub == 2 && c->pair2 && noRing && !fsurf;
     // Several steps per launch (k_steps).
     const bool tileSet = is_adj(q.op) ? c->tileAdjSet : c->tileFwdSet;
-    multi = (!is_born(q.op) || q.op == Op::BornFwd || q.op == Op::BornAdj) && noRing && !fsurf && !tileSet &&
-            c->spb == 1 && c->occ == 6 && p.minPad <= kStepsPadMax && wide_grid_ok(p.nz, p.nx) && !pair2 && !adj2;
+    multi = noRing && !fsurf && !tileSet && c->spb == 1 && c->occ == 6 && p.minPad <= kStepsPadMax &&
+            wide_grid_ok(p.nz, p.nx) && !pair2 && !adj2;
     // The lockstep kernel moves less than two passes on the largest tile: two
     // passes take 0.87 of its time for 1 shot of 200 x 400, but 1.04 for 4 and
     // 1.2 for 10.
@@ -372,8 +372,8 @@ void Call::plan_batches()
     if (multi && !lockstep) {
         const long any = 1L << 40;
         if (is_born(q.op)) stepsSrc = steps_config(B, win ? 1700 : any);
-        if (q.op != Op::BornAdj) steps = steps_config(B, q.op == Op::BornFwd && !win ? any : 1000);
-        else if (win && c->batchRec == 0) steps = steps_config(B, 3000);
+        if (q.op == Op::BornAdj && win && c->batchRec == 0) steps = steps_config(B, 3000);
+        if (q.op == Op::BornFwd || !is_born(q.op)) steps = steps_config(B, q.op == Op::BornFwd && !win ? any : 1000);
     }
     if (pairSlices == 4 && !pair2 && !adj2 && steps < 0 && stepsSrc < 0) {
         pairSlices = 2;
@@ -740,8 +740,8 @@ void Call::pass_pair2()
 // by fine step t and the scattered field by step t - 2.
 void Call::pass_lockstep()
 {
-    HIPC(launch_fill(pairs, (long)nb * 2 * nzx, s));
-    HIPC(launch_fill(pairsQ, (long)nb * 2 * nzx, s));
+    HIPC(launch_fill(pairs, (long)nb * pairSlices * nzx, s));
+    HIPC(launch_fill(pairsQ, (long)nb * pairSlices * nzx, s));
     const int T = p.ntw - 1;   // fine steps of each propagation
     auto ring3 = [&](long k) { return (k % 3) * nzx; };
     int curS = 1, curQ = 1;
@@ -1037,7 +1037,7 @@ void Call::passes_tomo()
     // once coarse sample k is complete.
     auto forward_pass = [&](unsigned mode, const ShotSlot* on, int ssKind, const ShotSlot* from, const float* scale,
                             int capture, const std::function<void(int)>& done) {
-        HIPC(launch_fill(pairs, (long)nb * 2 * nzx, s));
+        HIPC(launch_fill(pairs, (long)nb * pairSlices * nzx, s));
         StepArgs x = a;
         x.slots = on;
         x.cur = 1;
@@ -1106,7 +1106,7 @@ void Call::passes_tomo()
     // into the ring; done(k) once coarse sample k is complete.
     auto backward_pass = [&](int ssKind, const ShotSlot* from, const float* scale,
                              const std::function<void(int)>& done) {
-        HIPC(launch_fill(pairs, (long)nb * 2 * nzx, s));
+        HIPC(launch_fill(pairs, (long)nb * pairSlices * nzx, s));
         HIPC(launch_fill(cap, (long)nb * capSlices * nzx, s));
         StepArgs y = a;
         y.slots = dSlotsC;
@@ -1186,7 +1186,7 @@ void Call::passes_tomo()
         };
     };
     if (dataInput) {   // receiver wavefield R into P (computeTomoRecWfld, :1481-1515)
-        HIPC(launch_fill(pairs, (long)nb * 2 * nzx, s));
+        HIPC(launch_fill(pairs, (long)nb * pairSlices * nzx, s));
         StepArgs x = a;
         x.slots = dSlotsQ;
         x.cur = 1;
