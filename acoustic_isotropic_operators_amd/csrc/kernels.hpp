@@ -108,10 +108,10 @@ struct ExtBatch {
     int lagDir;             // +1 or -1
     int nts;                // coarse samples of W (bounds check of the time-lag batches)
 };
-using ExtBatchArgs = ExtBatch<kExtBatchMax>;
+struct ExtBatchArgs : ExtBatch<kExtBatchMax> {};
 // Time lags and the imaging of ext.hip take twice as many.
 constexpr int kTimeBatchMax = 2 * kExtBatchMax;
-using TimeBatchArgs = ExtBatch<kTimeBatchMax>;
+struct TimeBatchArgs : ExtBatch<kTimeBatchMax> {};
 
 // Image accumulation over a batch of coarse samples (k_img_acc_batch):
 // X.img += X.W[xOff[j]] * Y.W[yOff[j]] for j = 0 .. nk-1, in that order.
