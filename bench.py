@@ -265,7 +265,7 @@ def main():
         "dtype": "f32",
         "data": "synthetic",
         "config": {"workload": w.name, "shots": w.nShot, "grid": "500x1200 (padded %dx%d)" % (p["nz"], p["nx"]),
-                   "nts": p["nts"], "sub": p["sub"], "shots_per_launch_adj": info["batch"], "tile": a.tile or "32x16 forward, 32x32 adjoint", "lanes": lanes,
+                   "nts": p["nts"], "sub": p["sub"], "shots_per_launch_adj": info["batch"], "tile": a.tile or "64x32 forward, 32x32 adjoint", "lanes": lanes,
                    "inputs": "model/data/image resident in HBM"},
         "job_roofline_frac": job_bytes / t / 1e9 / HBM_PEAK_GBS,
         "shot_latency_ms": {"p50": float(np.percentile(lat, 50)) if lat else None,
