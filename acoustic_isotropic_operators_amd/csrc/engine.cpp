@@ -580,9 +580,23 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
     const bool fused = c->wide && maxSrcRing == 0;
     const bool multi = fused && maxRecRing == 0 && p.minPad <= kStepsPadMax;   // several steps per launch
     // 16 shots per batch by default, 8 per lane: at 400 x 1000 with 8 per
-    // batch a lane's launch covers the GPU about once (MI355X: 230 against
-    // 254 Gpts/s for 16; 12 and 32 gave 249 and 251).
-    int B = c->batchAdj > 0 ? c->batchAdj : (c->batchReq > 0 ? c->batchReq : 16);
+    // batch a lane's launch of one step covers the GPU about once (MI355X: 230
+    // against 254 Gpts/s for 16; 12 and 32 gave 249 and 251).  Several steps
+    // per launch are at their best with 1280 workgroups of 64 x 64 on, five
+    // rounds of the GPU: the shots are then split evenly into batches of that
+    // many, which also halves W.  Batches of 4 / 8 / 16 shots, misfit and
+    // gradient: 32 shots of 400 x 1000 (1296 workgroups for 8), 800 samples,
+    // 305 / 289 / 292 ms; 16 of 500 x 1200 (1680 for 8), 300 samples, 83.4 /
+    // 78.4 / 83.5 ms; 8 of 400 x 1000, 86.0 / 81.4 ms.
+    int B = c->batchAdj > 0 ? c->batchAdj : c->batchReq;
+    if (B <= 0) {
+        B = 16;
+        if (multi) {
+            const long wg = (long)((p.nz - 2 * kFat + 63) / 64) * ((p.nx - 2 * kFat + 63) / 64);
+            const int least = (int)std::min<long>(B, (1280 + wg - 1) / wg), batches = std::max(1, nShot / least);
+            B = std::min(B, (nShot + batches - 1) / batches);
+        }
+    }
     size_t freeB = 0, totalB = 0;
     HIPC(hipMemGetInfo(&freeB, &totalB));
     freeB += c->pairs.n + c->pairsQ.n + c->W.n + c->img.n + c->dreg.n + c->sig.n + c->ss.n + c->ck.n;

@@ -97,3 +97,18 @@ def test_born_passes(nzi, nxi, shots, sub, nts, pad):
     img = np.zeros((c.nx, c.nz), np.float32)
     ctx.born_adjoint(img, dr, srcs, wav, recs)
     np.testing.assert_array_equal(img, O.born_adjoint(g, c.vel, osrc, [wav], orec, dr, "f"))
+
+
+@pytest.mark.parametrize("nzi,nxi,shots", [(640, 832, 10), (640, 832, 21), (640, 832, 1), (2064, 2576, 2)])
+def test_gradient_batches(nzi, nxi, shots):
+    """The velocity gradient's own split into batches gives the bits of one
+    batch of all shots: one batch, several of equal and of unequal sizes, and
+    a batch for each shot."""
+    c, ctx, rng, srcs, recs, _, _ = _setup(nzi, nxi, shots, 2, 12, 20, 9)
+    m = rng.standard_normal((1, 1, c.nts)).astype(np.float32)
+    d = rng.standard_normal((shots, recs[0].nDev, c.nts)).astype(np.float32)
+    one, split = (np.zeros(c.vel.shape, np.float32) for _ in range(2))
+    ctx.nl_velocity_gradient(m, d, split, srcs, recs)
+    ctx.set_option("batchAdj", shots)
+    ctx.nl_velocity_gradient(m, d, one, srcs, recs)
+    assert np.any(one) and np.array_equal(one, split)
