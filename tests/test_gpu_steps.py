@@ -112,3 +112,18 @@ def test_gradient_batches(nzi, nxi, shots):
     ctx.set_option("batchAdj", shots)
     ctx.nl_velocity_gradient(m, d, one, srcs, recs)
     assert np.any(one) and np.array_equal(one, split)
+
+
+@pytest.mark.parametrize("nts", [2, 3, 17, 60])
+def test_gradient_first_and_later_calls(nts):
+    """A context's first velocity gradient, in short segments, and the later
+    ones, in as few as fit, give the bits of one segment per step."""
+    c, ctx, rng, srcs, recs, _, _ = _setup(48, 80, 2, 2, nts, 20, 9)
+    m = rng.standard_normal((1, 1, c.nts)).astype(np.float32)
+    d = rng.standard_normal((2, recs[0].nDev, c.nts)).astype(np.float32)
+    first, second, third, ref = (np.zeros(c.vel.shape, np.float32) for _ in range(4))
+    for g, every in ((first, 0), (second, 0), (ref, 1), (third, 0)):
+        ctx.nl_velocity_gradient(m, d, g, srcs, recs, checkpoint_every=every)
+    for g in (first, second, third):
+        assert np.array_equal(g, ref)
+    assert nts < 60 or np.any(ref)      # the waves have met
