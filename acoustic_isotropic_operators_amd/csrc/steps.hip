@@ -146,8 +146,14 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
                 else if (a.first[k]) ow[k / 2] = ld4s(G(S.W) + (a.its[k] + 1) * a.wStep, ooff, a.ntW);
             }
         }
-        if constexpr (WIN && !ADJ)
-            if (a.mtil) mt = ld4(G(a.mtil), ooff);
+        if constexpr (WIN) {
+            // from memory: the LDS copy of the old slice is overwritten by the
+            // first step, in other threads, with no barrier before it
+            ro = ld4(G(S.p[2 * a.pair + 1]), ooff);
+            rc = ld4(G(S.p[2 * a.pair]), ooff);
+            if constexpr (!ADJ)
+                if (a.mtil) mt = ld4(G(a.mtil), ooff);
+        }
         if constexpr (CAP) {
             if (!a.first[0] || a.its[0] > 0) cA = ld4(G(S.W) + a.its[0] * a.wStep, ooff);
             if (!a.first[0]) cB = ld4(G(S.W) + (a.its[0] + 1) * a.wStep, ooff);
@@ -190,12 +196,6 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
             if (j <= last) acc[j] = rd[ADJ ? -j : j];
     }
     __syncthreads();
-    if constexpr (WIN) {
-        if (own) {
-            rc = *(const f4a*)&(odd ? P1 : P0)[oli];
-            ro = *(const f4a*)&(odd ? P0 : P1)[oli];
-        }
-    }
     const bool sponge = z0 - HZ < a.minPad || x0 - E < a.minPad || z0 + TZ + HZ > nzi - a.minPad || x0 + TX + E > nxi - a.minPad;
 
     auto step = [&](auto KS, auto SPONGE) {
