@@ -524,8 +524,8 @@ static int grad_steps_config(const aiso_ctx* c, int nShot)
 // keep p_{t-1} itself and image in a kernel of its
 // own, which makes the Laplacian again; with them every segment is
 // recomputed.  Misfit and gradient of 8 shots of 400 x 1000 points, 800 samples
-// (MI355X): 132 ms with those and K = 40, 95 ms with one segment, 77 ms with
-// three steps per launch.
+// (MI355X): 131 ms with those and K = 40; one segment 95 ms, 80 ms with three
+// steps per launch; 101 ms with those in segments of 80.
 void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dataGrad, float* velGrad,
                  aiso_device* const* srcs, int nShot, aiso_device* const* recs, int nRec, int every, int mem)
 {
@@ -600,21 +600,18 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
     size_t freeB = 0, totalB = 0;
     HIPC(hipMemGetInfo(&freeB, &totalB));
     freeB += c->pairs.n + c->pairsQ.n + c->W.n + c->img.n + c->dreg.n + c->sig.n + c->ss.n + c->ck.n;
-    // Steps per segment.  Every segment but the last is propagated twice, so
-    // the fused kernels take as few as a quarter of the free memory, at most
-    // 64 GB, holds slices for (one where it holds every step's).  Allocating
-    // that much costs up to 30 ms per GB, where the driver has no cleared
-    // memory left: a context's first gradient, which may be its only one,
-    // takes segments of 2 sqrt(T) steps, 3 sqrt(T) slices with the checkpoints
-    // (as many as segments of sqrt(T) steps need).  8 shots of 400 x 1000, 800 samples: 2.3 GB, 102 ms with the
-    // misfit; 30 GB, 80 ms, and 0 to 1.7 s for the allocation.
+    // Steps per segment.  Every segment but the last is propagated twice; with
+    // segments of 2 sqrt(T) steps, W and the checkpoints hold 3 sqrt(T) slices,
+    // as many as the unfused kernels' segments of sqrt(T) steps take.  Longer
+    // ones are the caller's choice (checkpointEvery): they save up to the
+    // recompute, but hold more memory and may wait for it.  Misfit and gradient
+    // of 8 shots of 400 x 1000, 800 samples (T = 1598): K = 80 (2.3 GB) 101 ms,
+    // 800 (15 GB) 92 ms, T (30 GB) 80 ms, the first time up to 30 ms more per
+    // GB where the driver has no cleared memory left.
     int K = every > 0 ? std::min(every, T) : std::max(1, (int)std::ceil(std::sqrt((double)T)));
     if (every == 0 && fused) {
-        const size_t cap = c->gradAgain ? std::min<size_t>(freeB / 4, (size_t)64 << 30) : 0;
-        const long fit = (long)(cap / ((size_t)std::min(B, nShot) * nzx * 4));
-        const int Kmax = (int)std::min<long>(T, std::max<long>(2 * K, fit)), segments = (T + Kmax - 1) / Kmax;
+        const int Kmax = std::min(T, 2 * K), segments = (T + Kmax - 1) / Kmax;
         K = (T + segments - 1) / segments;
-        c->gradAgain = true;
     }
     const int nSeg = (T - 1) / K + 1;                  // segments start at t = 0, K, 2K, ... < T
     const int nCk = fused ? nSeg - 1 : nSeg;           // of which these are started from checkpoints

@@ -143,7 +143,6 @@ struct aiso_ctx {
     size_t stageOff = 0;
     hipEvent_t stageEv = nullptr;
     bool stagePending = false;
-    bool gradAgain = false;          // a velocity gradient was made: the next one takes W in few segments
     // Lanes: the shots of a batch split over streams whose kernels run
     // concurrently, so one lane's launch tail (CUs idle while its last
     // workgroups finish) and launch gap are filled by the other's.  On

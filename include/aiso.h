@@ -246,10 +246,12 @@ aiso_status aiso_nl_forward_noalloc(aiso_ctx* ctx, int add, const float* model, 
  * model: the source signals of aiso_nl_forward ([nShotSig][nSrcDev][nts]);
  * dataGrad: dJ/d(data) [nShot][nRec][nts]; velGrad (out): dJ/d(velocity)
  * on the padded grid [nx][nz], overwritten.  checkpointEvery: fine steps
- * between checkpoints (0: as many as a quarter of the free device memory, at
- * most 64 GB, holds slices for, at least ceil(sqrt(ntw - 1)); a gradient
- * whose steps all fit recomputes nothing).  mem applies to dataGrad
- * and velGrad (the model is read through the host either way). */
+ * between checkpoints, T = ntw - 1 at most (0: at most 2 ceil(sqrt(T)), in
+ * segments of equal length, or ceil(sqrt(T)) where a source lies in the FAT
+ * ring or the caller chose a tile, a register budget or shots per workgroup).
+ * Per shot the context holds that many slices and two for each checkpoint; a
+ * gradient whose steps are one segment recomputes nothing.  mem applies to
+ * dataGrad and velGrad (the model is read through the host either way). */
 aiso_status aiso_nl_velocity_gradient(aiso_ctx* ctx, const float* model, int nShotSig,
                                       const float* dataGrad, float* velGrad,
                                       aiso_device* const* sources, int nShot,
