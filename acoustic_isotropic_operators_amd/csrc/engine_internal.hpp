@@ -219,6 +219,10 @@ struct Request {
     int mem;
 };
 
+// Bytes of W up to which a Born forward of two fine steps per sample may leave
+// its lockstep form.
+constexpr size_t kTwoPassBytes = (size_t)1 << 30;
+
 // What a call steps on, for its choice of tile: the kernels of the nonlinear
 // passes and their velocity gradient, the lockstep Born pass, the other Born
 // passes, or the extended and tomographic ones.

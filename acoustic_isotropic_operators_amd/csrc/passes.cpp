@@ -281,6 +281,13 @@ void Call::build_geometry()
 void Call::plan_batches()
 {
     lockstep = q.op == Op::BornFwd && p.sub == 2 && c->lockstep;
+    // Shots per launch: an explicit request, else as many as keep the `hot`
+    // slices every fine step touches (per shot) within the on-die cache
+    // budget; never more than device memory holds.
+    const int byDir = is_adj(q.op) ? c->batchAdj : c->batchFwd, asked = byDir > 0 ? byDir : c->batchReq;
+    auto cached = [&](int hot) {
+        return std::min((int)std::max<long>(4, c->cacheBudget / ((long)hot * nzx * 4)), 32);
+    };
     // Two fine steps per launch (k_fwd_pair2, k_rec2) when no source or
     // receiver point lies in the FAT ring, whose values those kernels take as 0.
     bool noRing = true;
@@ -294,8 +301,19 @@ void Call::plan_batches()
             wide_grid_ok(p.nz, p.nx) && !pair2 && !adj2;
     // The lockstep kernel moves less than two passes on the largest tile: two
     // passes take 0.87 of its time for 1 shot of 200 x 400, but 1.04 for 4 and
-    // 1.2 for 10.
-    if (multi && lockstep && steps_config(std::min(q.nShot, 32), 0) >= 0) lockstep = false;
+    // 1.2 for 10.  They hold nts slices of W where lockstep holds three, so
+    // only short records leave it: a launch's W has to fit 1 GiB and an eighth
+    // of the free memory.
+    if (multi && lockstep) {
+        const int most = asked > 0 ? asked : cached(2);
+        const int batches = (q.nShot + most - 1) / most, shots = (q.nShot + batches - 1) / batches;
+        const size_t bytes = (size_t)shots * p.nts * nzx * 4;
+        if (steps_config(shots, 0) >= 0 && bytes <= kTwoPassBytes) {
+            size_t freeB = 0, totalB = 0;
+            HIPC(hipMemGetInfo(&freeB, &totalB));
+            lockstep = bytes > (freeB + c->W.n) / 8;
+        }
+    }
     pairSlices = pair2 || adj2 || (multi && !lockstep) ? 4 : 2;
     wSlices = lockstep ? 3 : p.nts;
     needW = is_born(q.op);
@@ -334,11 +352,7 @@ void Call::plan_batches()
     if (needImg) perShot += (size_t)nImg * nzx * 4;
     if (tomo) perShot += (size_t)(p.nts + capSlices) * nzx * 4;   // scattered / receiver wavefield + captures
     c->bytesPerShot = perShot;
-    // Shots per launch: an explicit request, else as many as keep the
-    // slices every fine step touches (per shot) within the on-die cache
-    // budget; never more than device memory holds.
-    B = is_adj(q.op) ? c->batchAdj : c->batchFwd;
-    if (B <= 0) B = c->batchReq;
+    B = asked;
     if (B <= 0) {
         int hot = 2;                                  // wavefield pair
         if (lockstep) hot = 7;                        // two pairs + secondary-source ring
@@ -346,8 +360,7 @@ void Call::plan_batches()
         else if (q.op == Op::ExtFwd) hot = 4;         // + two secondary-source slices
         else if (q.op == Op::ExtAdj) hot = 3;         // + receiver slice (the image is touched once per extK samples)
         else if (tomo) hot = 4;                       // + secondary source and captured slices
-        B = (int)std::max<long>(4, c->cacheBudget / ((long)hot * nzx * 4));
-        B = std::min(B, 32);
+        B = cached(hot);
     }
     {
         size_t freeB = 0, totalB = 0;
