@@ -1019,6 +1019,7 @@ aiso_status aiso_ctx_set_option(aiso_ctx* c, const char* key, int value)
         else if (k == "extBatch") {
             if (value < 1 || value > kExtBatchMax) throw Error(AISO_ERR_PARAM, "extBatch must be 1..16");
             c->extBatch = value;
+            c->extBatchSet = true;
         }
         else if (k == "lanes") {
             if (value < 1 || value > 4) throw Error(AISO_ERR_PARAM, "lanes must be 1..4");

@@ -151,6 +151,7 @@ struct aiso_ctx {
     int lanes = 2;
     bool lanesSet = false;              // the caller chose them
     int extBatch = 16;                  // coarse samples per offset-imaging / secondary-source launch
+    bool extBatchSet = false;           // the caller chose them
     int curLanes = 1;                   // lanes of the call in progress
     std::vector<hipStream_t> lane;
     hipEvent_t forkEv = nullptr;

@@ -328,7 +328,9 @@ void Call::plan_batches()
     // as often (10 shots of 400 x 1000, 21 offsets, 400 samples: 38.9 ms against
     // 41.6 with 16).
     wideImg = q.op == Op::ExtAdj && !tlag && p.hExt > kOffsetSsMin && p.hExt <= kOffsetSsMax && wide_grid_ok(p.nz, p.nx);
-    extK = std::min((is_ext(q.op) && tlag && p.hExt <= 10) || wideImg ? 2 * c->extBatch : c->extBatch, p.nts);
+    // Either only where the caller left the batch open: it bounds the ring.
+    const bool twice = !c->extBatchSet && ((is_ext(q.op) && tlag && p.hExt <= 10) || wideImg);
+    extK = std::min(twice ? 2 * c->extBatch : c->extBatch, p.nts);
     ssSlices = is_ext(q.op) || tomo ? extK + 1 : 2;
     needImg = q.op == Op::BornAdj || q.op == Op::ExtAdj || q.op == Op::TomoAdj || wemva;
     // captured coarse samples kept per shot: the WEMVA forward's imaging and

@@ -117,7 +117,9 @@ aiso_status aiso_ctx_set_tile(aiso_ctx* ctx, int tz, int tx);
  *       image per shot, model [nShot][nExt][nx][nz], instead of their sum
  *       (for callers that batch independent requests; default 0);
  *   "extBatch" 1..16: coarse samples per offset-imaging / secondary-source
- *       launch of the extended Born operators (default 16);
+ *       launch of the extended operators, which hold one slice more per shot
+ *       (default 16, and 32 until it is set for extended Born calls of up to
+ *       21 time lags and adjoints of 13 to 21 offsets);
  *   "lanes" 1..4: streams the shots of a launch are split over, whose
  *       kernels run concurrently (default 2; the extended, tomographic and
  *       WEMVA operators and the two-step kernels run on one);
