@@ -17,8 +17,8 @@ at once, each on its own context and HIP stream, so their kernels overlap on
 the device.  Whenever a slot is free, the oldest pending request picks the
 batch key (model, kind, reflectivity); every pending request with that key
 joins it, up to ``max_shots`` and up to what the HBM budget admits (the
-engine's bytes per shot of that kind on that model times the shots, see
-below).  A request that arrives while calls run is admitted as soon as a
+engine's bytes per shot of that kind on that model times the shots, and its
+bytes per call, see below).  A request that arrives while calls run is admitted as soon as a
 slot and memory free up: it does not wait for the running calls to finish.
 When nothing runs, the oldest request is admitted even if it alone exceeds
 the budget (the engine itself splits a call into launches that fit the free
@@ -93,14 +93,23 @@ class _Model:
         first.ctx = self.new_context()     # the velocity checks run when the model is added
         self.slots = [first]
         self.active = 0                    # calls running on this model
-        nzx = p["nz"] * p["nx"]
-        traces = 4 * p["nts"] * (self.rec[0].nDev + 8)
-        # engine bytes per shot by kind: wavefield pairs, the Born forward's
-        # lockstep ring, the adjoints' nts source slices, offset ring and image
-        self.bytes_per_shot = {"nl_forward": 4 * nzx * 2 + traces,
-                               "born_forward": 4 * nzx * (2 + (5 if p["sub"] == 2 else p["nts"])) + traces,
-                               "born_adjoint": 4 * nzx * (2 + p["nts"] + 2 + 1) + traces,
-                               "bornext_adjoint": 4 * nzx * (2 + p["nts"] + 17 + nExt) + traces}
+        nzx, nts, sub = p["nz"] * p["nx"], p["nts"], p["sub"]
+        traces = 4 * nts * (self.rec[0].nReg + 4 * sub)          # a point source has at most four grid points
+        # Engine bytes per shot by kind: two pairs of slices per field
+        # (several steps per launch), the Born forward's lockstep ring, the
+        # adjoints' nts source slices, offset ring and image.
+        ring = min(self.options.get("extBatch", 32 if 6 <= (nExt - 1) // 2 <= 10 else 16), nts) + 1
+        lockstep = sub == 2 and self.options.get("lockstep", 1)
+        born = (11 if self.options.get("pair2") else 7) if lockstep else 4 + nts
+        self.bytes_per_shot = {"nl_forward": 4 * nzx * 4 + traces,
+                               "born_forward": 4 * nzx * born + traces,
+                               "born_adjoint": 4 * nzx * (4 + nts + 2 + 1) + traces,
+                               "bornext_adjoint": 4 * nzx * (4 + nts + ring + nExt) + traces}
+        # Bytes that a call takes beyond those of its shots: a short Born
+        # forward of few points keeps every source slice, at most 1 GiB and
+        # the shots whose 64 x 32 tiles number 256.
+        tiles = -(-(p["nz"] - 10) // 64) * -(-(p["nx"] - 10) // 32)
+        self.bytes_per_call = {"born_forward": min(1 << 30, 256 // tiles * 4 * nzx * nts) if lockstep else 0}
 
     def new_context(self):
         ctx = A.Context(self.params, self.device)
@@ -206,8 +215,8 @@ class Server:
             slot = _Slot()
         else:
             return None
-        bps = m.bytes_per_shot[key[1]]
-        room = self.budget - self.resident_bytes + slot.reserved
+        bps, once = m.bytes_per_shot[key[1]], getattr(m, "bytes_per_call", {}).get(key[1], 0)
+        room = self.budget - self.resident_bytes + slot.reserved - once
         cap = min(self.max_shots, int(room // bps))
         if cap < 1:
             if self.running:
@@ -216,7 +225,7 @@ class Server:
         batch = [r for r in self.queue if self._key(r) == key][:cap]
         taken = set(map(id, batch))
         self.queue = collections.deque(r for r in self.queue if id(r) not in taken)
-        need = bps * len(batch)
+        need = bps * len(batch) + once
         if need > slot.reserved:
             self.resident_bytes += need - slot.reserved
             slot.reserved = need
