@@ -594,11 +594,12 @@ aiso_status aiso_batch_get_config(const aiso_batch* b, int* tz, int* tx, int* wi
                                   int* lanes, int* graph)
 {
     if (!b) return AISO_ERR_PARAM;
-    if (tz) *tz = b->cfg.tz;
-    if (tx) *tx = b->cfg.tx;
-    if (windowsPerLaunch) *windowsPerLaunch = b->cfg.spl;
-    if (blocksPerCU) *blocksPerCU = b->cfg.persist;
-    if (lanes) *lanes = b->cfg.lanes;
+    const aiso::BatchConfig c = run_config(b);
+    if (tz) *tz = c.tz;
+    if (tx) *tx = c.tx;
+    if (windowsPerLaunch) *windowsPerLaunch = c.spl;
+    if (blocksPerCU) *blocksPerCU = c.persist;
+    if (lanes) *lanes = c.lanes;
     if (graph) *graph = b->useGraph;
     return AISO_OK;
 }

@@ -348,9 +348,12 @@ aiso_status aiso_batch_set_windows(aiso_batch* b, int nWin, const int* nz, const
  * of that many per CU, each looping over tiles); lanes 1..4: streams the
  * launch groups alternate over, whose kernels run concurrently (default 2);
  * graph != 0: capture each group's time loop in a HIP graph on first use
- * and replay it later. */
+ * and replay it later.  Until a configuration is set or tuned, a call runs 32
+ * x 32 tiles in two groups where its windows have 4096 such tiles, else 32 x
+ * 16 tiles in one. */
 aiso_status aiso_batch_set_config(aiso_batch* b, int tz, int tx, int windowsPerLaunch, int blocksPerCU, int lanes,
                                   int graph);
+/* The configuration that a call runs. */
 aiso_status aiso_batch_get_config(const aiso_batch* b, int* tz, int* tx, int* windowsPerLaunch, int* blocksPerCU,
                                   int* lanes, int* graph);
 /* Autotuner: times `steps` fine steps of every launch group, on its lanes,
