@@ -2672,6 +2672,7 @@ hipError_t launch_ext_ss_batch(const ExtBatchArgs& a, int nshots, hipStream_t s)
         const dim3 g(xcd_padded(bx * by * bz)), b(kExtTZ, 4);
         if (a.hExt <= 2) hipLaunchKernelGGL(k_ext_ss_tile<2>, g, b, 0, s, a, nshots, bx, by, bz);
         else if (a.hExt <= 5) hipLaunchKernelGGL(k_ext_ss_tile<5>, g, b, 0, s, a, nshots, bx, by, bz);
+        else if (a.hExt <= 10) hipLaunchKernelGGL(k_ext_ss_tile<10>, g, b, 0, s, a, nshots, bx, by, bz);   // grids of 2^30 points on
         else hipLaunchKernelGGL(k_ext_ss_tile<20>, g, b, 0, s, a, nshots, bx, by, bz);
     } else {
         dim3 g((nzi + 63) / 64, nshots, nxi);
@@ -2731,12 +2732,13 @@ hipError_t launch_tomo_adj_ss(const ExtBatchArgs& a, int nshots, hipStream_t s)
     const int nzi = a.nz - 2 * FAT, nxi = a.nx - 2 * FAT;
     if (nzi <= 0 || nxi <= 0) return hipSuccess;
     if (a.hExt > kOffsetSsMin && a.hExt <= kOffsetSsMax && wide_grid_ok(a.nz, a.nx)) return launch_offset_ss_tomo(a, nshots, s);
-    if (a.hExt <= kOffsetSsMin) {
+    if (a.hExt <= 10) {
         const int bx = (nxi + kExtTX - 1) / kExtTX, by = (nshots + kExtSsSpb - 1) / kExtSsSpb;
         const int bz = (nzi + kExtTZ - 1) / kExtTZ;
         const dim3 g(xcd_padded(bx * by * bz)), b(kExtTZ, 4);
         if (a.hExt <= 2) hipLaunchKernelGGL(k_tomo_adj_ss_tile<2>, g, b, 0, s, a, nshots, bx, by, bz);
-        else hipLaunchKernelGGL(k_tomo_adj_ss_tile<5>, g, b, 0, s, a, nshots, bx, by, bz);
+        else if (a.hExt <= 5) hipLaunchKernelGGL(k_tomo_adj_ss_tile<5>, g, b, 0, s, a, nshots, bx, by, bz);
+        else hipLaunchKernelGGL(k_tomo_adj_ss_tile<10>, g, b, 0, s, a, nshots, bx, by, bz);   // grids of 2^30 points on
     } else {
         hipLaunchKernelGGL(k_tomo_adj_ss, column_grid(a.nz, a.nx, nshots), dim3(64), 0, s, a);
     }
