@@ -51,14 +51,14 @@ def build_lib():
         obj = os.path.join(bdir, src.replace(".", "_") + ".o")
         lang = [] if src.endswith(".hip") else ["-x", "hip"]
         # the kernels' register, scratch and occupancy figures, kept for the tests
-        remarks = ["-Rpass-analysis=kernel-resource-usage"] if src == "kernels.hip" else []
+        remarks = ["-Rpass-analysis=kernel-resource-usage"] if src.endswith(".hip") else []
         cmds.append([HIPCC, *HIP_FLAGS, *remarks, *lang, "-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
     # one compiler per object, side by side (each is single-threaded)
     with ThreadPoolExecutor(max_workers=min(len(cmds), max(1, (os.cpu_count() or 1) // 2))) as ex:
         results = list(ex.map(_run, cmds))
     with open(RESOURCE_USAGE, "w") as f:
-        f.write(results[0].stderr)
+        f.write("".join(r.stderr for r, o in zip(results, objs) if o.endswith("_hip.o")))
     out = os.path.join(PKG, "libaiso.so")
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", out, *objs])
     return out

@@ -185,14 +185,15 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
     // a recorder's cells: its ascends by at most one per step, so samples
     // its[0] .. its[0] + K; the adjoint's are columns of sig
     gf* rd = nullptr;
-    float acc[K + 1];
+    constexpr int NA = ADJ ? K : K + 1;
+    float acc[NA];
     const int last = ADJ ? a.n - 1 : a.its[a.n - 1] - a.its[0] + 1;
     if (r0 + t < r1) {
         const int2 en = re[r0 + t];
         ri = en.x;
         rd = ADJ ? G(S.sig) + ((long)en.y * a.ntw + a.itw[0]) : G(S.dreg) + ((long)en.y * a.nts + a.its[0]);
 #pragma unroll
-        for (int j = 0; j <= K; ++j)
+        for (int j = 0; j < NA; ++j)
             if (j <= last) acc[j] = rd[ADJ ? -j : j];
     }
     __syncthreads();
@@ -389,7 +390,10 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
         if constexpr (!REC) return;
         if (ri >= 0) {
 #pragma unroll
-            for (int k = 0; k < K; ++k) rv[k] = k == i ? n[ri] : rv[k];
+            for (int k = 0; k < K; ++k) {
+                if constexpr (ADJ) acc[k] = k == i ? acc[k] + n[ri] : acc[k];
+                else rv[k] = k == i ? n[ri] : rv[k];
+            }
         }
         for (int k = r0 + t + NTH; k < r1; k += NTH) {
             const int2 en = re[k];
@@ -419,12 +423,10 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
         }
     }
     if (ri >= 0) {
+        if constexpr (!ADJ) {
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-            if (k >= a.n) continue;
-            if constexpr (ADJ) {
-                acc[k] += rv[k];
-            } else {
+            for (int k = 0; k < K; ++k) {
+                if (k >= a.n) continue;
 #pragma unroll
                 for (int j = 0; j < K; ++j)
                     if (j == a.its[k] - a.its[0]) {
@@ -434,7 +436,7 @@ __global__ __launch_bounds__(NTH) void k_steps(const StepsArgs a)
             }
         }
 #pragma unroll
-        for (int j = 0; j <= K; ++j)
+        for (int j = 0; j < NA; ++j)
             if (j <= last) rd[ADJ ? -j : j] = acc[j];
     }
 }
