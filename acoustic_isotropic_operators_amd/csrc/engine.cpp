@@ -622,6 +622,7 @@ void run_nl_grad(aiso_ctx* c, const float* model, int nShotSig, const float* dat
     B = std::min(B, nShot);
     c->batchUsed = B;
     const int steps = multi ? grad_steps_config(c, B) : -1, nSl = steps >= 0 ? 4 : 2;   // slices per field
+    c->kernels = kernels_used(c, steps);
     float* pairs = (float*)c->pairs.need((size_t)B * nSl * nzx * 4);
     float* pairsA = (float*)c->pairsQ.need((size_t)B * nSl * nzx * 4);
     float* W = (float*)c->W.need((size_t)B * K * nzx * 4);
@@ -1078,6 +1079,7 @@ aiso_status aiso_ctx_get_option(const aiso_ctx* c, const char* key, int* value)
         else if (k == "occupancy") *value = c->occ;
         else if (k == "cacheBudgetMB") *value = (int)(c->cacheBudget >> 20);
         else if (k == "profileEvery") *value = c->profEvery;
+        else if (k == "kernels") *value = c->kernels;
         else throw Error(AISO_ERR_PARAM, "unknown option " + k);
     });
 }

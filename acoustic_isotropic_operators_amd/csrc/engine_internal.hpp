@@ -111,6 +111,7 @@ struct aiso_ctx {
     int tzFwd = 32, txFwd = 16, tzAdj = 32, txAdj = 32;
     bool tileFwdSet = false, tileAdjSet = false;   // the caller chose the tile
     bool wide = false;                  // the call in progress steps on the wide kernels (wide.hip)
+    int kernels = 0;                    // kernels of the last call's main pass: kernels_used
     int streamNT = 1;
     size_t bytesPerShot = 0;
     // work buffers
@@ -230,6 +231,9 @@ constexpr size_t kTwoPassBytes = (size_t)1 << 30;
 enum class TileUse { NlFwd, NlAdj, NlGrad, Lockstep, Fwd, Adj, FwdGeneric, AdjGeneric };
 // Sets the tile of a call (c->tz, c->tx) and whether it runs on the wide kernels.
 void select_tile(aiso_ctx* c, TileUse use, int nShot);
+// What aiso_ctx_get_option("kernels") reports of a pass that runs on k_steps
+// configuration `steps`, or on one step per launch (-1).
+inline int kernels_used(const aiso_ctx* c, int steps) { return steps >= 0 ? 2 + steps : c->wide ? 1 : 0; }
 int tiles_z(const aiso_ctx* c);
 int tiles_x(const aiso_ctx* c);
 struct TileLists {

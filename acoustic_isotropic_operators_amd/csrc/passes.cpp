@@ -390,6 +390,7 @@ void Call::plan_batches()
         if (q.op == Op::BornAdj && win && c->batchRec == 0) steps = steps_config(B, 3000);
         if (q.op == Op::BornFwd || !is_born(q.op)) steps = steps_config(B, q.op == Op::BornFwd && !win ? any : 1000);
     }
+    c->kernels = kernels_used(c, steps);
     if (pairSlices == 4 && !pair2 && !adj2 && steps < 0 && stepsSrc < 0) {
         pairSlices = 2;
         c->bytesPerShot -= 2 * nzx * 4;

@@ -134,7 +134,10 @@ aiso_status aiso_ctx_set_tile(aiso_ctx* ctx, int tz, int tx);
  *       aiso_ctx_wavefield; parfile keys saveWavefield / wavefieldShotNumber
  *       of F/src/BornShotsGpu.cpp:18-19). */
 aiso_status aiso_ctx_set_option(aiso_ctx* ctx, const char* key, int value);
-/* The current value of an aiso_ctx_set_option knob (tiles as tz * 100 + tx). */
+/* The current value of an aiso_ctx_set_option knob (tiles as tz * 100 + tx),
+ * or "kernels": those of the main pass of the last nonlinear or Born call or
+ * velocity gradient: 0 one point per lane, 1 four points per lane, 2 / 3 / 4
+ * several steps per launch on 32 x 32 / 64 x 32 / 64 x 64 tiles. */
 aiso_status aiso_ctx_get_option(const aiso_ctx* ctx, const char* key, int* value);
 /* Derived sizes: ntw, sub, nShotsPerLaunch actually used by the last call. */
 aiso_status aiso_ctx_info(const aiso_ctx* ctx, int* ntw, int* batchUsed, size_t* bytesPerShot);
