@@ -77,8 +77,8 @@ def parse():
     return ap.parse_args()
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_fwd_pair_born_lsrtm_80x500x1200_hbm_traffic.md")
-KERNEL_SRC = os.path.join(ROOT, "acoustic_isotropic_operators_amd", "csrc", "kernels.hip")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_wide_pair_born_lsrtm_80x500x1200_hbm_traffic.md")
+KERNEL_SRC = os.path.join(ROOT, "acoustic_isotropic_operators_amd", "csrc", "wide.hip")   # k_wide_pair
 
 
 def _sha16(path):
@@ -91,7 +91,7 @@ def measured_traffic():
     """Fabric bytes per launch of the lockstep Born forward kernel from the
     committed FETCH_SIZE / WRITE_SIZE summary (copy-calibrated), with the
     summary's file name; the figure is used only when the summary was taken
-    on the kernels.hip in this tree (its KERNELS_SHA16 line), else None."""
+    on the kernel source in this tree (its KERNELS_SHA16 line), else None."""
     vals = {}
     try:
         for line in open(TRAFFIC_FILE):
@@ -102,7 +102,7 @@ def measured_traffic():
         return None, "no counter summary"
     src = os.path.relpath(TRAFFIC_FILE, ROOT)
     if vals.get("KERNELS_SHA16") != _sha16(KERNEL_SRC):
-        return None, f"{src} was taken on another kernels.hip"
+        return None, f"{src} was taken on another {os.path.basename(KERNEL_SRC)}"
     try:
         return float(vals["TRAFFIC_BYTES_PER_LAUNCH"]), src
     except (KeyError, ValueError):
