@@ -45,7 +45,9 @@ void hip_check(hipError_t e, const char* what)
 //   free surface     0.87-0.98 from 1 shot of 200 x 400 points to 20 of 500 x 1200, every pass
 //   Born lockstep    1.01 at 80 workgroups, 0.96 at 240, 0.91-0.93 from 640 on
 //   nonlinear        1.04-1.13 to 1640 workgroups, 0.96 at 3492, 0.85-0.87 from 16000 on
-//   its adjoint      0.89-0.95 to 1968 workgroups, 1.01-1.09 from 16000 on
+//   its adjoint      0.89-0.95 to 1968 workgroups, 1.01-1.09 from 16000 on; the calls below the
+//                    line that k_steps leaves: a source or receiver in the FAT ring, grids under
+//                    about 100 points wide
 //   its gradient     0.96 (8 shots of 400 x 1000)
 // The nonlinear passes of few shots are bound by each workgroup's latency,
 // which four points per lane lengthen; the adjoint's loads of v2dt2 for its

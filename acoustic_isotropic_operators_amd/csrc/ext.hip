@@ -6,7 +6,9 @@
 // sample, 168 of them the products and sums; no LDS conflicts).  All offsets
 // are computed without a test, those beyond 2 hExt on zeros: with a branch per
 // offset every LDS read was waited for.  64 x 32 tiles stage 2.25 times their
-// points, the one-point kernels' 64 x 16 ones 3.5 times.
+// points, the one-point kernels' 64 x 16 ones 3.5 times.  Not built for more
+// than 21 offsets: the model values of 41 would take 164 registers and leave
+// one workgroup per CU; that form was not measured.
 // Extended forward, 6 shots of 500 x 1200, 21 offsets, 300 samples: 27.2 ms,
 // one point per lane 30.3; tomographic adjoint, 6 shots of 300 x 700: 33.1 ms,
 // 37.1.  Up to 11 offsets both take the same time, and the one-point kernels

@@ -275,9 +275,11 @@ void Call::build_geometry()
 
 // Shots per launch and the passes' forms: the Born forward with sub == 2
 // runs its two propagations in lockstep (the secondary source then lives in
-// a 3-slice ring instead of nts slices); with a free surface the nonlinear
-// and Born passes run the surface instances of the specialized kernels
-// (k_step_fs, k_fwd_pair_fs), without two steps per launch.
+// a 3-slice ring instead of nts slices), or in two passes where those take
+// several fine steps per launch; with a free surface every pass of the
+// nonlinear and Born operators takes one step per launch, on the wide kernels
+// or, where the caller chose a tile, a register budget or shots per workgroup,
+// the surface instances of the one-point kernels (k_step_fs, k_fwd_pair_fs).
 void Call::plan_batches()
 {
     lockstep = q.op == Op::BornFwd && p.sub == 2 && c->lockstep;
@@ -340,11 +342,11 @@ void Call::plan_batches()
     // when sub == 2, so captures and imaging are written once per coarse
     // step instead of accumulated at every fine step.
     win = p.sub == 2;
-    // The extended-Born, tomographic and WEMVA operators, and every pass with
-    // a free surface, step on the unspecialized kernel.  A GPU run of the
-    // specialized kernel on the extended-Born path ended in a memory fault
-    // whose cause was never shown; the specialized kernel is not built for
-    // the extended modes.
+    // The extended-Born, tomographic and WEMVA operators step on the
+    // unspecialized kernel, but for source passes that take several steps per
+    // launch.  A GPU run of the specialized kernel on the extended-Born path
+    // ended in a memory fault whose cause was never shown; the specialized
+    // kernel is not built for the extended modes.
     generic = is_ext(q.op) || tomo;
 
     size_t perShot = pairSlices * nzx * 4 + (size_t)nRecRegMax * p.nts * 4 + (size_t)nSrcRegMax * p.ntw * 4;

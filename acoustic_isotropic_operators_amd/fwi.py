@@ -5,8 +5,10 @@ float32 tensor) to the data of the nonlinear operator [nShot][nRec][nts]
 through ``torch.autograd``:
 
 * forward: ``aiso_nl_forward`` with the tensor as the context's velocity;
-* backward: ``aiso_nl_velocity_gradient``, the adjoint-state gradient with
-  checkpointed forward recomputation, given the incoming dL/d(data).
+* backward: ``aiso_nl_velocity_gradient``, the adjoint-state gradient, given
+  the incoming dL/d(data).  It propagates the source field again, in segments
+  of at most 2 sqrt(T) of its T fine steps, all but the last of them twice
+  (from checkpoints); ``checkpoint_every=`` sets another length.
 
 The reference's FWI drives ``nonlinearFwiPropShotsGpu`` with pySolver and
 takes the Born adjoint as the gradient (PY/fwiMain.py:123-142,

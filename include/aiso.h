@@ -91,10 +91,12 @@ aiso_status aiso_ctx_set_velocity(aiso_ctx* ctx, const float* vel, int mem);
 
 /* Shots advanced together by one launch (0 = automatic, by free HBM). */
 aiso_status aiso_ctx_set_batch(aiso_ctx* ctx, int shotsPerLaunch);
-/* Tile shape of the time-step kernel for forward and adjoint calls: tz in
- * {32,64}, tx in {16,32} (default 32 x 16 forward, 32 x 32 adjoint; the
- * extended, tomographic and WEMVA forwards, and forwards with a free
- * surface, default to 32 x 32 until a tile is set). */
+/* Tile shape of the one-point-per-lane step kernels for forward and adjoint
+ * calls: tz in {32,64}, tx in {16,32}.  Until a tile is set, the engine picks
+ * kernels and tile by the operator and the points of a launch: several steps
+ * per launch, four points per lane, or one on 32 x 16 (forward) or 32 x 32
+ * tiles (adjoint, and the extended, tomographic and WEMVA forwards).  A caller
+ * that sets a tile takes the last; results are the same bits. */
 aiso_status aiso_ctx_set_tile(aiso_ctx* ctx, int tz, int tx);
 /* Engine tuning knobs by name (no counterpart in the reference):
  *   "streamNT" 0/1: non-temporal access to the coarse wavefield stream;
@@ -104,7 +106,8 @@ aiso_status aiso_ctx_set_tile(aiso_ctx* ctx, int tz, int tx);
  *       and adjoint when sub == 2 and no device lies in the FAT ring;
  *   "batchFwd", "batchAdj": shots per launch of forward / adjoint calls
  *       (0 = aiso_ctx_set_batch's value, or automatic; "batchAdj" also
- *       sets the batch of aiso_nl_velocity_gradient, 16 by default);
+ *       sets the batch of aiso_nl_velocity_gradient, by default 16, or as few
+ *       as fill the GPU five times where it takes several steps per launch);
  *   "batchRec": group size of the adjoint receiver pass within a batch;
  *   "shotsPerBlock" 1/2: shots advanced by one workgroup of the step kernel;
  *   "occupancy" 0/6/8: the specialized step kernels compiled to the
@@ -121,8 +124,10 @@ aiso_status aiso_ctx_set_tile(aiso_ctx* ctx, int tz, int tx);
  *       (default 16, and 32 until it is set for extended Born calls of up to
  *       21 time lags and adjoints of 13 to 21 offsets);
  *   "lanes" 1..4: streams the shots of a launch are split over, whose
- *       kernels run concurrently (default 2; the extended, tomographic and
- *       WEMVA operators and the two-step kernels run on one);
+ *       kernels run concurrently (default 2, and 1 until it is set where a
+ *       step of the launch is under 1.3 million points; the two-step kernels,
+ *       and passes of several steps per launch on at most 256 workgroups, run
+ *       on one);
  *   "leg1", "leg2" 0/1: legs of the tomographic operator (parfile keys
  *       leg1/leg2 of F/src/tomoExtGpu.cpp:10-11, default 1);
  *   "sloth" 0/1: time-lag extended Born model is a slowness-squared
